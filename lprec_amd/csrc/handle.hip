@@ -3,13 +3,13 @@
 // lpRgpu (src/include/lpRgpu.cuh:6-81, src/cuda/lpRgpu.cu, params.cu,
 // gridStorage.cu) behind the C ABI of include/lprec_amd.h.
 #include <algorithm>
-#include <array>
 #include <climits>
 #include <cmath>
 #include <complex>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -87,14 +87,15 @@ struct lp_handle {
     // fwd, rows inv, cols) and their launch shapes
     int rtc_mode = 1;
     int rtc_cols_req = 0;   // threads of the compiled column pass (0: automatic)
-    // variant of the compiled passes: k_cols_ct VAR (bits 0-1), at least 4
-    // waves per SIMD (bit 2), odd-radix output pairs per item 4 instead of 8 (bit 3)
+    // variant of the compiled passes: index arithmetic redone per slice (bit
+    // 1), at least 4 waves per SIMD (bit 2); bits 0 and 3 have no effect
     int rtc_cols_var = 14;
-    int rtc_pp = 0;   // output pairs per odd-radix work item of the loaded module
-    bool rtc_tried = false;
-    hipModule_t rtc_mod = nullptr;
+    bool rtc_tried = false;       // with the current settings ...
+    bool rtc_pair_tried = false;  // ... and the filtered pair pass
+    std::vector<hipModule_t> rtc_mods;
     void* rtc_fn[4] = {nullptr, nullptr, nullptr, nullptr};   // + the filtered sinogram pair pass
     int rtc_R = 0, rtc_rows_nt = 0, rtc_cols_nt = 0, rtc_pair_nt = 0;
+    float* d_wodd = nullptr;   // matrix-core DFT weights of the compiled passes
     size_t lds_limit = 65536;
     std::string err;
     std::vector<void*> allocs;
@@ -244,7 +245,7 @@ struct lp_handle {
     ~lp_handle() {
         DeviceGuard g(device);
         prof_clear();
-        if (rtc_mod) (void)hipModuleUnload(rtc_mod);
+        for (hipModule_t m : rtc_mods) (void)hipModuleUnload(m);
         for (void* p : allocs) (void)hipFree(p);
     }
 };
@@ -779,12 +780,6 @@ std::string csrc_dir() {
     return (k == std::string::npos ? std::string(".") : p.substr(0, k)) + "/csrc";
 }
 
-std::string radix_list(const FftPlan& p) {
-    std::string r;
-    for (int i = 0; i < p.nst; ++i) r += ", " + std::to_string(p.radix[i]);
-    return r;
-}
-
 struct RtcCode {
     std::vector<char> code;
     std::vector<std::string> lowered;
@@ -792,9 +787,8 @@ struct RtcCode {
 std::mutex g_rtc_mu;
 std::map<std::string, std::shared_ptr<RtcCode>> g_rtc_cache;
 
-std::shared_ptr<RtcCode> rtc_compile(const std::string& arch, int pp, const std::vector<std::string>& names,
-                                     std::string& err) {
-    std::string key = arch + ";" + std::to_string(pp);
+std::shared_ptr<RtcCode> rtc_compile(const std::string& arch, const std::vector<std::string>& names, std::string& err) {
+    std::string key = arch;
     for (const auto& n : names) key += ";" + n;
     std::lock_guard<std::mutex> lock(g_rtc_mu);
     auto it = g_rtc_cache.find(key);
@@ -808,11 +802,11 @@ std::shared_ptr<RtcCode> rtc_compile(const std::string& arch, int pp, const std:
         return nullptr;
     }
     for (const auto& n : names) hiprtcAddNameExpression(prog, n.c_str());
-    const std::string a = "--offload-arch=" + arch, inc = "-I" + dir, dpp = "-DLPCT_ODD_PP=" + std::to_string(pp);
+    const std::string a = "--offload-arch=" + arch, inc = "-I" + dir;
     // packed FP32 instructions off, as for the library's own kernels
-    const char* opts[] = {a.c_str(), "-O3", "-std=c++17", inc.c_str(), dpp.c_str(),
+    const char* opts[] = {a.c_str(), "-O3", "-std=c++17", inc.c_str(),
                           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"};
-    if (hiprtcCompileProgram(prog, 9, opts) != HIPRTC_SUCCESS) {
+    if (hiprtcCompileProgram(prog, 8, opts) != HIPRTC_SUCCESS) {
         size_t n = 0;
         hiprtcGetProgramLogSize(prog, &n);
         std::string log(n, '\0');
@@ -846,52 +840,156 @@ std::shared_ptr<RtcCode> rtc_compile(const std::string& arch, int pp, const std:
 
 bool pow2_in(int n, int lo, int hi) { return n >= lo && n <= hi && (n & (n - 1)) == 0; }
 
-// Output pairs per odd-radix work item (LPCT_ODD_PP of fft_ct.hpp, one value
-// per compiled module) from 4, 6 and 8: the fewest cycles over the module's
-// passes, counting for each radix R > 5 the rounds of the block's threads
-// over its work items (lines x M/R butterflies x ceil(hR/PP) groups) times
-// the pairs per item (hR = (R-1)/2 terms each).  E.g. the 4128-point column
-// at 512 threads: PP 4 -> 576 items, two rounds of 4; PP 6 -> 384, one of 6.
-int odd_pairs(const std::vector<std::array<int, 4>>& passes, const std::vector<const FftPlan*>& plans) {
-    int best = 4;
-    long long best_cost = LLONG_MAX;
-    for (int pp : {4, 6, 8}) {
-        long long cost = 0;
-        for (size_t k = 0; k < passes.size(); ++k) {
-            const int M = passes[k][0], NL = passes[k][1], NT = passes[k][2], weight = passes[k][3];
-            const FftPlan& pl = *plans[k];
-            for (int i = 0; i < pl.nst; ++i) {
-                const int R = pl.radix[i];
-                if (R <= 5 || !(R & 1)) continue;
-                const int hR = (R - 1) / 2;
-                const int P = hR <= 2 ? 2 : (hR <= pp ? ((hR + 1) & ~1) : pp);
-                const long long items = (long long)NL * (M / R) * ((hR + P - 1) / P);
-                cost += weight * ((items + NT - 1) / NT) * P * hR;
-            }
-        }
-        if (cost < best_cost) { best_cost = cost; best = pp; }
+// Radix sequence and block size of one compiled pass (FFTs of NL lines of M
+// points per block, fft_ct.hpp).
+struct CtPlan {
+    std::vector<int> radix;
+    int nt = 0;
+    bool ok() const { return nt > 0; }
+};
+
+// VALU operations per point of a register butterfly of radix r (0: not one of
+// the register radices): reads, writes and index arithmetic, the twiddle
+// product, and about two operations per radix-2 level, p per factor p > 3.
+double ct_radix_ops(int r) {
+    double ops = 15;
+    for (int p : {2, 3, 5, 7, 11, 13})
+        while (r % p == 0) { ops += p == 2 ? 2 : p == 3 ? 4 : p; r /= p; }
+    return r == 1 ? ops : 0;
+}
+
+// Chooses the plan with the fewest VALU operations over all lanes, idle ones
+// included: stages cost much the same per point whatever their radix, so few
+// large ones win, as long as a thread's butterflies of a stage fit in
+// registers (32 points) and the butterflies fill the block's threads.  Prime
+// factors >= 17 are matrix-core stages and come first (no twiddles), then the
+// odd radices (their strided LDS writes spread over the banks).  Blocks that
+// would leave a CU under 12 waves are charged for the latency they expose.
+// Measured at M = 4128, 32 slices: 43 12 8 on 384 threads against 43 8 4 3 on
+// 512 of the former out-of-place kernels (DESIGN table).
+CtPlan ct_plan(int M, int NL, size_t lds_line, size_t lds_limit, int force_nt) {
+    CtPlan best;
+    if (NL * lds_line > lds_limit) return best;
+    std::vector<int> primes;
+    int C = M;
+    for (int q = 2; (long long)q * q <= C; ++q)
+        while (C % q == 0) { primes.push_back(q); C /= q; }
+    if (C > 1) primes.push_back(C);
+    std::vector<int> big;
+    C = 1;
+    for (int q : primes) {
+        if (q >= 17) big.push_back(q);
+        else C *= q;
     }
+    if (C < 2) return best;
+    std::sort(big.rbegin(), big.rend());
+    double best_cost = 0;
+    std::vector<int> cur;
+    auto consider = [&](int nt) {
+        // staging and stores, whatever the lanes: more in the row passes (R2C step, transposed access)
+        double cost = (double)NL * M * (NL > 1 ? 30 : 10);
+        const double waves = nt / 64.0;
+        for (int R : big) {
+            const long long cols = (long long)NL * (M / R), ntl = (cols + 15) / 16;
+            const int mt = ((R - 1) / 2 + 16) / 16, ks = ((R - 1) / 2 + 4) / 4;
+            double unit = 0;
+            for (int mtc = 1; mtc <= std::min(mt, 4); ++mtc) {
+                const long long units = ntl * ((mt + mtc - 1) / mtc);
+                const double ju = std::ceil(units / waves);
+                if (ju * mtc > 6) continue;   // accumulators: 16 registers each
+                // per step 4 mtc matrix instructions (8 VALU slots each, partly hidden) and ~16 VALU
+                const double c = waves * 64 * ju * ks * (4.0 * mtc * 8 * 0.6 + 16);
+                if (unit == 0 || c < unit) unit = c;
+            }
+            if (unit == 0) return;
+            cost += unit + 60.0 * nt;
+        }
+        for (int r : cur) {
+            const long long items = (long long)NL * (M / r), ni = (items + nt - 1) / nt;
+            if (ni * r > 24) return;
+            // above 16 points the butterfly's temporaries crowd the registers
+            cost += (double)nt * ni * r * ct_radix_ops(r) * (r > 16 ? 1.2 : 1.0) + 60.0 * nt;
+        }
+        // the waves of a CU's blocks hide each other's latency, up to 16 (128 registers)
+        const double blocks = std::min(std::floor(160.0 * 1024 / (NL * lds_line)), std::floor(16 / waves));
+        cost *= std::pow(16 / std::max(blocks * waves, 1.0), 0.8);
+        if (!best.ok() || cost < best_cost) {
+            best_cost = cost;
+            best.radix = big;
+            // odd radices first, largest first
+            std::vector<int> rest = cur;
+            std::sort(rest.begin(), rest.end(), [](int a, int b) { return (a & 1) != (b & 1) ? (a & 1) > (b & 1) : a > b; });
+            best.radix.insert(best.radix.end(), rest.begin(), rest.end());
+            best.nt = nt;
+        }
+    };
+    // every factorisation of C into register radices (non-increasing)
+    std::function<void(int, int)> walk = [&](int n, int top) {
+        if (n == 1) {
+            if (force_nt) consider(force_nt);
+            else for (int nt : {64, 128, 192, 256, 384, 512, 768, 1024}) consider(nt);
+            return;
+        }
+        for (int r = std::min(n, top); r >= 2; --r)
+            if (n % r == 0 && ct_radix_ops(r) > 0) {
+                cur.push_back(r);
+                walk(n / r, r);
+                cur.pop_back();
+            }
+    };
+    walk(C, 24);
     return best;
 }
 
-// threads of a mixed-radix pass over `points` values (as threads_for)
-int rtc_threads(long long points) {
-    int nt = 256;
-    while (points > 16LL * nt && nt < 1024) nt *= 2;
-    return nt;
+std::string radix_args(const CtPlan& p) {
+    std::string r;
+    for (int q : p.radix) r += ", " + std::to_string(q);
+    return r;
+}
+
+// LDS slots of a line of M points under the plan (slots() of fft_ct.hpp)
+int ct_slots(const CtPlan& p, int M) { return (p.radix[0] & 1) ? M : M + (M >> 4) + 1; }
+
+// Weights of the matrix-core stages (mfma_stage of fft_ct.hpp) of the prime
+// factors >= 17 of M, largest first: per tile of 16 outputs p and step of 4
+// terms q, 64 cosines then 64 sines of 2 pi p q / R in lane order (lane l:
+// output l mod 16, term l / 16), zero outside p, q <= (R - 1) / 2.
+std::vector<float> ct_weights(int M) {
+    std::vector<int> big;
+    for (int q = 2; (long long)q * q <= M; ++q)
+        while (M % q == 0) { if (q >= 17) big.push_back(q); M /= q; }
+    if (M >= 17) big.push_back(M);
+    std::sort(big.rbegin(), big.rend());
+    std::vector<float> w;
+    for (int R : big) {
+        const int hR = (R - 1) / 2, mt = (hR + 16) / 16, ks = (hR + 4) / 4;
+        for (int m = 0; m < mt; ++m)
+            for (int k = 0; k < ks; ++k)
+                for (int part = 0; part < 2; ++part)
+                    for (int l = 0; l < 64; ++l) {
+                        const int p = m * 16 + (l & 15), q = k * 4 + (l >> 4);
+                        const double t = 2.0 * M_PI * (double)(((long long)p * q) % R) / R;
+                        w.push_back(p <= hR && q <= hR ? (float)(part ? std::sin(t) : std::cos(t)) : 0.f);
+                    }
+    }
+    return w;
 }
 
 void rtc_build(lp_handle* h) {
-    if (h->rtc_tried || !h->rtc_mode) return;
-    h->rtc_tried = true;
-    if (h->rtc_mod) {
-        (void)hipModuleUnload(h->rtc_mod);
-        h->rtc_mod = nullptr;
+    if (!h->rtc_mode) return;
+    if (!h->rtc_tried) {
+        for (hipModule_t m : h->rtc_mods) (void)hipModuleUnload(m);
+        h->rtc_mods.clear();
         h->rtc_fn[0] = h->rtc_fn[1] = h->rtc_fn[2] = h->rtc_fn[3] = nullptr;
+        h->rtc_pair_tried = false;
     }
-    const bool rows = !pow2_in(h->h, 256, 4096), cols = !pow2_in(h->Nr, 256, 4096);
-    // the filtered pair pass has no register kernel at any length
-    const bool pair = h->has_filter;
+    const bool rows = !h->rtc_tried && !pow2_in(h->h, 256, 4096), cols = !h->rtc_tried && !pow2_in(h->Nr, 256, 4096);
+    // the filtered pair pass has no register kernel at any length; when the
+    // filter comes after the first build (lp_init_adj after lp_init_fwd), it
+    // is a module of its own
+    const bool pair = h->has_filter && !h->rtc_pair_tried;
+    h->rtc_tried = true;
+    if (pair) h->rtc_pair_tried = true;
     if (!rows && !cols && !pair) return;
     const char* v = std::getenv("LPREC_AMD_VERBOSE");
     const bool verbose = v && v[0] == '1';
@@ -899,57 +997,76 @@ void rtc_build(lp_handle* h) {
     if (hipGetDeviceProperties(&prop, h->device) != hipSuccess) return;
     std::string arch(prop.gcnArchName);
     arch = arch.substr(0, arch.find(':'));
-    // rows per block of the compiled row passes: at most 8 (the generic
-    // kernels' limit) and few enough that their two LDS buffers fit
-    int R = std::min(h->R, 8);
-    while (R > 1 && 2 * (size_t)lds_slots(R * row_ldm(h, R)) * sizeof(float2) > h->lds_limit) R /= 2;
-    const int ldm = row_ldm(h, R);
-    const int rnt = rtc_threads((long long)R * h->h);
-    const int cnt = h->rtc_cols_req ? h->rtc_cols_req : rtc_threads(h->Nr);
-    const std::string hr = radix_list(h->plan_h), mr = radix_list(h->plan_M);
-    const std::string wpe = (h->rtc_cols_var & 4) ? "4" : "2";
-    const int pnt = rtc_threads(2LL * h->N);
+    // waves per SIMD the registers are budgeted for: what the blocks' LDS lets
+    // a CU hold, up to 4 (128 registers)
+    auto wpe = [&](size_t lds, int nt) {
+        if (!(h->rtc_cols_var & 4)) return std::string("2");
+        const int waves = (int)(160 * 1024 / lds) * (nt / 64);
+        return std::to_string(std::max(2, std::min(4, waves / 4)));
+    };
+    const std::string opq = (h->rtc_cols_var & 2) ? "1" : "0";
     // only the passes this handle runs (slot: 0 rows fwd, 1 rows inv, 2 cols,
     // 3 filtered sinogram pair)
     std::vector<std::string> names;
     std::vector<int> slot;
-    if (rows) {
-        const std::string args = std::to_string(h->h) + ", " + std::to_string(R) + ", " + std::to_string(ldm) + ", " +
-                                 std::to_string(rnt) + ", " + wpe + ", 1" + hr + ">";
-        names.push_back("lpct::k_rows_fwd_ct<" + args);
-        slot.push_back(0);
-        names.push_back("lpct::k_rows_inv_ct<" + args);
-        slot.push_back(1);
-    }
-    if (cols) {
-        names.push_back("lpct::k_cols_ct<" + std::to_string(h->Nr) + ", " + std::to_string(cnt) + ", " + wpe + ", " +
-                        std::to_string(h->rtc_cols_var & 3) + mr + ">");
-        slot.push_back(2);
-    }
-    if (pair) {
-        names.push_back("lpct::k_sino_rows_pair_ct<" + std::to_string(h->N) + ", " + std::to_string(pnt) + ", " + wpe +
-                        radix_list(h->plan_2N) + ">");
-        slot.push_back(3);
-    }
-    // the passes of the module (length, lines per block, threads, launches
-    // per fwd or adj call) for the choice of output pairs per work item
-    std::vector<std::array<int, 4>> passes;
-    std::vector<const FftPlan*> plans;
-    if (rows) {
-        passes.push_back({h->h, R, rnt, 2});
-        plans.push_back(&h->plan_h);
-    }
-    if (cols) {
-        passes.push_back({h->Nr, 1, cnt, 1});
-        plans.push_back(&h->plan_M);
-    }
-    if (pair) {
-        passes.push_back({2 * h->N, 1, pnt, 1});
-        plans.push_back(&h->plan_2N);
-    }
+    int R = 0, rnt = 0, cnt = 0, pnt = 0;
     std::string err;
-    const int pp = (h->rtc_cols_var & 8) ? odd_pairs(passes, plans) : 8;
-    auto code = rtc_compile(arch, pp, names, err);
+    auto name = [&](int k, const std::string& n) {
+        names.push_back("lpct::" + n + ">");
+        slot.push_back(k);
+    };
+    if (rows) {
+        // 16 rows per block give 128-byte segments of the transposed spectra,
+        // while two blocks still share a CU; else 8 rows (64-byte segments)
+        CtPlan p;
+        int ls = 0;
+        for (R = std::min(h->R, 16); R >= 1; R /= 2) {
+            if (h->Nr % R) continue;
+            const size_t most = R > 8 ? std::min<size_t>(h->lds_limit, 80 * 1024) : h->lds_limit;
+            const size_t line = (size_t)(h->h + (h->h >> 4) + 32) * sizeof(float2);   // padded, with the row offset
+            p = ct_plan(h->h, R, line, most, 0);
+            if (p.ok()) break;
+        }
+        if (p.ok()) {
+            ls = ct_slots(p, h->h);
+            while (ls % 32 != (32 / R) % 32) ++ls;
+            rnt = p.nt;
+            const std::string args = std::to_string(h->h) + ", " + std::to_string(R) + ", " + std::to_string(ls) + ", " +
+                                     std::to_string(rnt) + ", " + wpe((size_t)R * ls * sizeof(float2), rnt) + ", " + opq + radix_args(p);
+            name(0, "k_rows_fwd_ct<" + args);
+            name(1, "k_rows_inv_ct<" + args);
+        } else {
+            err = "no plan for the row length";
+        }
+    }
+    if (cols) {
+        const CtPlan p = ct_plan(h->Nr, 1, (size_t)(h->Nr + (h->Nr >> 4) + 1) * sizeof(float2), h->lds_limit, h->rtc_cols_req);
+        if (p.ok()) {
+            cnt = p.nt;
+            name(2, "k_cols_ct<" + std::to_string(h->Nr) + ", " + std::to_string(cnt) + ", " +
+                        wpe(ct_slots(p, h->Nr) * sizeof(float2), cnt) + ", " +
+                        std::to_string(h->rtc_cols_var & 3) + radix_args(p));
+        } else {
+            err = "no plan for the column length";
+        }
+    }
+    if (pair) {
+        const CtPlan p = ct_plan(2 * h->N, 1, (size_t)(2 * h->N + (2 * h->N >> 4) + 1) * sizeof(float2), h->lds_limit, 0);
+        if (p.ok()) {
+            pnt = p.nt;
+            name(3, "k_sino_rows_pair_ct<" + std::to_string(h->N) + ", " + std::to_string(pnt) + ", " +
+                        wpe(ct_slots(p, 2 * h->N) * sizeof(float2), pnt) + radix_args(p));
+        } else {
+            err = "no plan for the filter length";
+        }
+    }
+    if (!h->d_wodd) {
+        // h, Nr and 2N are N times powers of two: they share their large primes
+        const std::vector<float> w = ct_weights(h->N);
+        if (!w.empty() && h->upload(&h->d_wodd, w)) return;
+    }
+    std::shared_ptr<RtcCode> code;
+    if (!names.empty()) code = rtc_compile(arch, names, err);
     hipModule_t mod = nullptr;
     if (code && hipModuleLoadData(&mod, code->code.data()) != hipSuccess) {
         (void)hipGetLastError();
@@ -972,16 +1089,17 @@ void rtc_build(lp_handle* h) {
         if (verbose) std::fprintf(stderr, "lprec_amd: run-time compiled passes unavailable (%s)\n", err.c_str());
         return;
     }
-    h->rtc_mod = mod;
-    for (int i = 0; i < 4; ++i) h->rtc_fn[i] = fn[i];
-    h->rtc_R = R;
-    h->rtc_rows_nt = rnt;
-    h->rtc_cols_nt = cnt;
-    h->rtc_pair_nt = pnt;
-    h->rtc_pp = pp;
+    h->rtc_mods.push_back(mod);
+    for (int i = 0; i < 4; ++i)
+        if (fn[i]) h->rtc_fn[i] = fn[i];
+    if (rows) {
+        h->rtc_R = R;
+        h->rtc_rows_nt = rnt;
+    }
+    if (cols) h->rtc_cols_nt = cnt;
+    if (pair) h->rtc_pair_nt = pnt;
     if (verbose)
-        for (const auto& n : names)
-            std::fprintf(stderr, "lprec_amd: run-time compiled pass: %s (odd-radix output pairs %d)\n", n.c_str(), pp);
+        for (const auto& n : names) std::fprintf(stderr, "lprec_amd: run-time compiled pass: %s\n", n.c_str());
 }
 
 }  // namespace
@@ -1355,7 +1473,6 @@ int lp_init_adj(lp_handle* h, const int32_t* pi, const float* pf) {
         h->has_filter = true;
     }
     h->has_adj = true;
-    if (h->has_filter) h->rtc_tried = false;   // (re)build with the filtered pair pass
     rtc_build(h);
     return LP_OK;
 }
@@ -1410,13 +1527,14 @@ static lpk::RowPass row_pass(lp_handle* h, int nz) {
     rp.fft16 = h->fft16;
     rp.in_rows = nullptr;
     rp.out_rows = nullptr;
-    const bool rtc = h->rtc_mode && h->rtc_mod;
+    const bool rtc = h->rtc_mode;
     rp.rtc_rows_fwd = rtc ? h->rtc_fn[0] : nullptr;
     rp.rtc_rows_inv = rtc ? h->rtc_fn[1] : nullptr;
     rp.rtc_cols = rtc ? h->rtc_fn[2] : nullptr;
     rp.rtc_R = h->rtc_R;
     rp.rtc_rows_nt = h->rtc_rows_nt;
     rp.rtc_cols_nt = h->rtc_cols_nt;
+    rp.wodd = h->d_wodd;
     return rp;
 }
 
@@ -1550,8 +1668,9 @@ int lp_adj(lp_handle* h, float* f, const float* R, int ns0, void* stream) {
     sp.tw2N = h->has_filter ? h->tw[2 * h->Lf] : nullptr;
     sp.plan2N = h->plan_2N;
     sp.tw2Nc = h->has_filter ? h->tw[2 * N] : nullptr;
-    sp.rtc_pair = h->rtc_mode && h->rtc_mod ? h->rtc_fn[3] : nullptr;
+    sp.rtc_pair = h->rtc_mode ? h->rtc_fn[3] : nullptr;
     sp.rtc_pair_nt = h->rtc_pair_nt;
+    sp.wodd = h->d_wodd;
     hipEvent_t* ev = h->prof_begin(1);
     auto mark = [&](int i) { if (ev) (void)hipEventRecord(ev[i], s); };
     mark(0);
@@ -1718,6 +1837,7 @@ int lp_adj_T(lp_handle* h, float* R, const float* f, int ns0, void* stream) {
     sp.tw2Nc = h->has_filter ? h->tw[2 * N] : nullptr;
     sp.rtc_pair = nullptr;
     sp.rtc_pair_nt = 0;
+    sp.wodd = nullptr;
     if (h->cubic) {
         lpk::launch_col_iir_T(acc, h->d_tmp, ns0, h->P, N, h->colchunk, s);
         lpk::launch_sino_rows_T(h->d_tmp, R, ns0, sp, true, s);
@@ -1921,7 +2041,7 @@ int lp_get_tuning(const lp_handle* h, int key, int* value) {
         case 7: *value = h->pt_ok ? h->polar_t : 0; return LP_OK;
         case 8: *value = h->staged; return LP_OK;
         case 9: *value = h->box_rule; return LP_OK;
-        case 10: *value = h->rtc_mode && h->rtc_mod ? 1 : 0; return LP_OK;
+        case 10: *value = h->rtc_mode && !h->rtc_mods.empty() ? 1 : 0; return LP_OK;
         case 11: *value = h->rtc_cols_nt; return LP_OK;
         case 12: *value = h->rtc_cols_var; return LP_OK;
         case 13: *value = h->pzgroup; return LP_OK;

@@ -1843,8 +1843,8 @@ void launch_rows_fwd(const RowPass& rp0, const float* F, const int2* range, hipS
     dim3 grid(rg.Nrho / rg.R, 3, (rg.nz + rg.zgroup - 1) / rg.zgroup);
     if (rg.rtc_rows_fwd) {
         void* args[] = {&rg, &F, &range};
-        if (hipModuleLaunchKernel((hipFunction_t)rg.rtc_rows_fwd, grid.x, grid.y, grid.z, rg.rtc_rows_nt, 1, 1, 0, s,
-                                  args, nullptr) == hipSuccess)
+        if (hipModuleLaunchKernel((hipFunction_t)rg.rtc_rows_fwd, grid.x * grid.y * grid.z, 1, 1, rg.rtc_rows_nt, 1, 1,
+                                  0, s, args, nullptr) == hipSuccess)
             return;
         (void)hipGetLastError();   // the generic kernel does the pass
         RowPass rn = rp;
@@ -1895,8 +1895,8 @@ void launch_rows_inv(const RowPass& rp0, float* G, const int2* wrange, hipStream
     dim3 grid(rg.Nrho / rg.R, 3, (rg.nz + rg.zgroup - 1) / rg.zgroup);
     if (rg.rtc_rows_inv) {
         void* args[] = {&rg, &G, &wrange};
-        if (hipModuleLaunchKernel((hipFunction_t)rg.rtc_rows_inv, grid.x, grid.y, grid.z, rg.rtc_rows_nt, 1, 1, 0, s,
-                                  args, nullptr) == hipSuccess)
+        if (hipModuleLaunchKernel((hipFunction_t)rg.rtc_rows_inv, grid.x * grid.y * grid.z, 1, 1, rg.rtc_rows_nt, 1, 1,
+                                  0, s, args, nullptr) == hipSuccess)
             return;
         (void)hipGetLastError();   // the generic kernel does the pass
         RowPass rn = rp;
@@ -1959,8 +1959,8 @@ void launch_cols(const RowPass& rp0, const FftPlan& planM, const float2* twM, co
     if (rp.rtc_cols) {
         RowPass rc = rp;
         void* args[] = {&rc, &twM, &fzT};
-        if (hipModuleLaunchKernel((hipFunction_t)rc.rtc_cols, grid.x, grid.y, grid.z, rc.rtc_cols_nt, 1, 1, 0, s, args,
-                                  nullptr) == hipSuccess)
+        if (hipModuleLaunchKernel((hipFunction_t)rc.rtc_cols, grid.x * grid.y * grid.z, 1, 1, rc.rtc_cols_nt, 1, 1, 0, s,
+                                  args, nullptr) == hipSuccess)
             return;
         (void)hipGetLastError();   // the generic kernel below does the pass
     }

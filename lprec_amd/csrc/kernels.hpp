@@ -88,6 +88,7 @@ struct SinoPrep {
     // rtc_kernels.hpp, rtc_pair_nt threads; null: the generic kernel)
     void* rtc_pair;
     int rtc_pair_nt;
+    const float* wodd;        // its matrix-core weights (see RowPass.wodd)
 };
 void launch_sino_rows(const float* R, float* Rc, int nz, const SinoPrep& sp, bool cubic, hipStream_t s);
 // y-direction prefilter of [nz][L][W] (columns), chunked with halo, in -> out
@@ -123,6 +124,10 @@ struct RowPass {
     void* rtc_rows_inv;
     void* rtc_cols;
     int rtc_R, rtc_rows_nt, rtc_cols_nt;
+    // DFT weights of the prime factors >= 17 of the lengths, largest first, in
+    // the lane order of the matrix-core stage (mfma_stage of fft_ct.hpp; null
+    // when the lengths have none)
+    const float* wodd;
 };
 // R2C along theta of the gathered log-polar grids F [3][nz][Nrho][Ntheta];
 // range [3][Nrho]: [lo, hi) theta bounds of the non-empty points of each row
