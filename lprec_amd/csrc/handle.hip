@@ -845,6 +845,7 @@ bool pow2_in(int n, int lo, int hi) { return n >= lo && n <= hi && (n & (n - 1))
 struct CtPlan {
     std::vector<int> radix;
     int nt = 0;
+    double cost = 0;
     bool ok() const { return nt > 0; }
 };
 
@@ -858,16 +859,19 @@ double ct_radix_ops(int r) {
     return r == 1 ? ops : 0;
 }
 
-// Chooses the plan with the fewest VALU operations over all lanes, idle ones
-// included: stages cost much the same per point whatever their radix, so few
-// large ones win, as long as a thread's butterflies of a stage fit in
-// registers (32 points) and the butterflies fill the block's threads.  Prime
-// factors >= 17 are matrix-core stages and come first (no twiddles), then the
-// odd radices (their strided LDS writes spread over the banks).  Blocks that
-// would leave a CU under 12 waves are charged for the latency they expose.
-// Measured at M = 4128, 32 slices: 43 12 8 on 384 threads against 43 8 4 3 on
-// 512 of the former out-of-place kernels (DESIGN table).
-CtPlan ct_plan(int M, int NL, size_t lds_line, size_t lds_limit, int force_nt) {
+// Chooses the plan of least estimated time for `blocks` blocks: the
+// instructions of one wave (stages cost much the same per point whatever
+// their radix, so few large ones win, as long as a thread's butterflies of a
+// stage fit in registers -- 24 points -- and the butterflies fill the
+// threads), times the rounds that the waves of all blocks take over the
+// chip.  Prime factors >= 17 are matrix-core stages and come first (no
+// twiddles), then the odd radices (their strided LDS writes spread over the
+// banks).  Waves that share a CU hide each other's latency, up to 16 (128
+// registers).  Measured against the neighbours of its choices (32 slices):
+// M = 4128 columns, 43 12 8 on 192 threads 2.60 ms, on 256 2.99, on 384 3.5,
+// 43 8 4 3 on 192 2.93; rows of h = 1032, 43 24 on 512 threads 1.41 inverse,
+// on 384 2.0; 320 or 576 threads (uneven waves per SIMD) 1.5-2 times slower.
+CtPlan ct_plan(int M, int NL, size_t lds_line, size_t lds_limit, double blocks, int force_nt) {
     CtPlan best;
     if (NL * lds_line > lds_limit) return best;
     std::vector<int> primes;
@@ -883,12 +887,12 @@ CtPlan ct_plan(int M, int NL, size_t lds_line, size_t lds_limit, int force_nt) {
     }
     if (C < 2) return best;
     std::sort(big.rbegin(), big.rend());
-    double best_cost = 0;
     std::vector<int> cur;
     auto consider = [&](int nt) {
-        // staging and stores, whatever the lanes: more in the row passes (R2C step, transposed access)
-        double cost = (double)NL * M * (NL > 1 ? 30 : 10);
+        if (nt > 64 && nt * 4 > NL * M) return;
         const double waves = nt / 64.0;
+        // staging and stores (in the row passes also the R2C step, transposed access)
+        double cost = (double)NL * M / nt * (NL > 1 ? 30 : 10);
         for (int R : big) {
             const long long cols = (long long)NL * (M / R), ntl = (cols + 15) / 16;
             const int mt = ((R - 1) / 2 + 16) / 16, ks = ((R - 1) / 2 + 4) / 4;
@@ -898,23 +902,24 @@ CtPlan ct_plan(int M, int NL, size_t lds_line, size_t lds_limit, int force_nt) {
                 const double ju = std::ceil(units / waves);
                 if (ju * mtc > 6) continue;   // accumulators: 16 registers each
                 // per step 4 mtc matrix instructions (8 VALU slots each, partly hidden) and ~16 VALU
-                const double c = waves * 64 * ju * ks * (4.0 * mtc * 8 * 0.6 + 16);
+                const double c = ju * ks * (4.0 * mtc * 8 * 0.6 + 16);
                 if (unit == 0 || c < unit) unit = c;
             }
             if (unit == 0) return;
-            cost += unit + 60.0 * nt;
+            cost += unit + 60 + 4 * waves;
         }
         for (int r : cur) {
             const long long items = (long long)NL * (M / r), ni = (items + nt - 1) / nt;
             if (ni * r > 24) return;
             // above 16 points the butterfly's temporaries crowd the registers
-            cost += (double)nt * ni * r * ct_radix_ops(r) * (r > 16 ? 1.2 : 1.0) + 60.0 * nt;
+            cost += (double)ni * r * ct_radix_ops(r) * (r > 16 ? 1.2 : 1.0) + 60 + 4 * waves;
         }
-        // the waves of a CU's blocks hide each other's latency, up to 16 (128 registers)
-        const double blocks = std::min(std::floor(160.0 * 1024 / (NL * lds_line)), std::floor(16 / waves));
-        cost *= std::pow(16 / std::max(blocks * waves, 1.0), 0.8);
-        if (!best.ok() || cost < best_cost) {
-            best_cost = cost;
+        const double cu_blocks = std::min(std::floor(160.0 * 1024 / (NL * lds_line)), std::floor(16 / waves));
+        const double cu_waves = std::max(cu_blocks * waves, 1.0);
+        // (independent blocks fill each other's barriers)
+        cost *= std::max(1.0, blocks * waves / (256 * 16.0) * std::pow(16 / cu_waves, 0.8)) * (1 + 0.3 / std::max(cu_blocks, 1.0));
+        if (!best.ok() || cost < best.cost) {
+            best.cost = cost;
             best.radix = big;
             // odd radices first, largest first
             std::vector<int> rest = cur;
@@ -1004,7 +1009,10 @@ void rtc_build(lp_handle* h) {
         const int waves = (int)(160 * 1024 / lds) * (nt / 64);
         return std::to_string(std::max(2, std::min(4, waves / 4)));
     };
-    const std::string opq = (h->rtc_cols_var & 2) ? "1" : "0";
+    // index arithmetic redone per slice; up to 256 points there are registers
+    // to hold it (and the twiddles, whose latency short kernels would expose):
+    // N = 256, 4 slices 104 -> 101 us; N = 528 the other way, 172 -> 586 us (spills)
+    auto opaque = [&](int M) { return M > 256 && (h->rtc_cols_var & 2) != 0; };
     // only the passes this handle runs (slot: 0 rows fwd, 1 rows inv, 2 cols,
     // 3 filtered sinogram pair)
     std::vector<std::string> names;
@@ -1016,23 +1024,26 @@ void rtc_build(lp_handle* h) {
         slot.push_back(k);
     };
     if (rows) {
-        // 16 rows per block give 128-byte segments of the transposed spectra,
-        // while two blocks still share a CU; else 8 rows (64-byte segments)
+        // rows per block: 16 give 128-byte segments of the transposed spectra
+        // (8 and 4: 64 and 32 bytes), fewer give a small batch more blocks
         CtPlan p;
         int ls = 0;
-        for (R = std::min(h->R, 16); R >= 1; R /= 2) {
-            if (h->Nr % R) continue;
-            const size_t most = R > 8 ? std::min<size_t>(h->lds_limit, 80 * 1024) : h->lds_limit;
-            const size_t line = (size_t)(h->h + (h->h >> 4) + 32) * sizeof(float2);   // padded, with the row offset
-            p = ct_plan(h->h, R, line, most, 0);
-            if (p.ok()) break;
+        const size_t line = (size_t)(h->h + (h->h >> 4) + 32) * sizeof(float2);   // padded, with the row offset
+        for (int r = std::min(h->R, 16); r >= 1; r /= 2) {
+            if (h->Nr % r || (p.ok() && r < 4)) continue;
+            CtPlan q = ct_plan(h->h, r, line, h->lds_limit, 3.0 * h->Ns * (h->Nr / r), 0);
+            if (3LL * h->Ns * h->Nr / r * q.nt > 256 * 1024) q.cost *= r >= 16 ? 1.0 : r >= 8 ? 1.04 : r >= 4 ? 1.25 : 2.0;
+            if (q.ok() && (!p.ok() || q.cost < p.cost)) {
+                p = q;
+                R = r;
+            }
         }
         if (p.ok()) {
             ls = ct_slots(p, h->h);
             while (ls % 32 != (32 / R) % 32) ++ls;
             rnt = p.nt;
             const std::string args = std::to_string(h->h) + ", " + std::to_string(R) + ", " + std::to_string(ls) + ", " +
-                                     std::to_string(rnt) + ", " + wpe((size_t)R * ls * sizeof(float2), rnt) + ", " + opq + radix_args(p);
+                                     std::to_string(rnt) + ", " + wpe((size_t)R * ls * sizeof(float2), rnt) + (opaque(h->h) ? ", 1" : ", 0") + radix_args(p);
             name(0, "k_rows_fwd_ct<" + args);
             name(1, "k_rows_inv_ct<" + args);
         } else {
@@ -1040,18 +1051,20 @@ void rtc_build(lp_handle* h) {
         }
     }
     if (cols) {
-        const CtPlan p = ct_plan(h->Nr, 1, (size_t)(h->Nr + (h->Nr >> 4) + 1) * sizeof(float2), h->lds_limit, h->rtc_cols_req);
+        const CtPlan p = ct_plan(h->Nr, 1, (size_t)(h->Nr + (h->Nr >> 4) + 1) * sizeof(float2), h->lds_limit,
+                                 3.0 * h->Ns * h->h, h->rtc_cols_req);
         if (p.ok()) {
             cnt = p.nt;
             name(2, "k_cols_ct<" + std::to_string(h->Nr) + ", " + std::to_string(cnt) + ", " +
                         wpe(ct_slots(p, h->Nr) * sizeof(float2), cnt) + ", " +
-                        std::to_string(h->rtc_cols_var & 3) + radix_args(p));
+                        (opaque(h->Nr) ? "2" : "0") + radix_args(p));
         } else {
             err = "no plan for the column length";
         }
     }
     if (pair) {
-        const CtPlan p = ct_plan(2 * h->N, 1, (size_t)(2 * h->N + (2 * h->N >> 4) + 1) * sizeof(float2), h->lds_limit, 0);
+        const CtPlan p = ct_plan(2 * h->N, 1, (size_t)(2 * h->N + (2 * h->N >> 4) + 1) * sizeof(float2), h->lds_limit,
+                                 0.5 * h->Ns * h->P0, 0);
         if (p.ok()) {
             pnt = p.nt;
             name(3, "k_sino_rows_pair_ct<" + std::to_string(h->N) + ", " + std::to_string(pnt) + ", " +
