@@ -323,10 +323,18 @@ __global__ void k_col_iir(const float* __restrict__ in, float* __restrict__ outp
 #pragma unroll
         for (int n = 0; n < NV; ++n) v[n] = (n & 1) ? 0.f : c0[(size_t)n * W];
     } else {
+        // rows clamped into the column, then masked: every load unconditional
+        // here too (the whole grid is edge chunks up to L = 48, and small
+        // launches are all latency: the stage 11.2 -> 9.8 us at N = 64, 1 slice)
+#pragma unroll
+        for (int n = 0; n < NV; ++n) v[n] = col[(size_t)min(max(r0 - K + n, 0), L - 1) * W];
+        __builtin_amdgcn_sched_barrier(0);   // (a select beside its load would wait for it)
+        int m = ((r0 - K) % stuff + stuff) % stuff;   // (r0 - K + n) mod stuff, uniform over the block
 #pragma unroll
         for (int n = 0; n < NV; ++n) {
-            int row = r0 - K + n;   // uniform over the block
-            v[n] = (row >= 0 && row < L && row % stuff == 0) ? col[(size_t)row * W] : 0.f;
+            const int row = r0 - K + n;
+            if (row < 0 || row >= L || m != 0) v[n] = 0.f;
+            m = m + 1 == stuff ? 0 : m + 1;
         }
     }
     const float zp = kPole;
@@ -2040,10 +2048,14 @@ __global__ void k_col_iir_T(const float* __restrict__ in, float* __restrict__ ou
     const float zp = kPole;
     const float kap = zp / (zp - 1.0f);
     float v[NV];
+    // rows clamped into the column, then masked: all loads in flight together
+#pragma unroll
+    for (int n = 0; n < NV; ++n) v[n] = col[(size_t)min(max(r0 - K + n, 0), L - 1) * W];
+    __builtin_amdgcn_sched_barrier(0);   // (a select beside its load would wait for it)
 #pragma unroll
     for (int n = 0; n < NV; ++n) {
-        int row = r0 - K + n;
-        v[n] = (row >= 0 && row < L) ? col[(size_t)row * W] : 0.f;
+        const int row = r0 - K + n;
+        if (row < 0 || row >= L) v[n] = 0.f;
     }
     // transposed anticausal stage: causal sweep (zeros before row 0 make the
     // first chunk exact), u = -z s, kap s at row L-1, nothing past it
