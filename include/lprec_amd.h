@@ -110,7 +110,8 @@ int lp_info(const lp_handle* h, int64_t* info);
  * key 1 = slices per block in the row/column passes (>=1; halved on launch
  * while a pass would have fewer than 2048 blocks), key 2 = rows per
  * prefilter column chunk (32, 64 or 128), key 3 = slices per block in the
- * tiled gathers (>=1), key 4 = FFT kernel family (1 = radix-16 register
+ * tiled gathers and scatters (>=1; halved on launch while there would be too
+ * few blocks, each kind by its own count), key 4 = FFT kernel family (1 = radix-16 register
  * kernels where the length is 16*k*16 with k in {1,2,4,8,16}; 2, the
  * default = the same with the inverse row pass at h = 1024 as a 32 x 32
  * register FFT with 32 lanes per row; 0 = the mixed-radix LDS kernels
@@ -140,8 +141,8 @@ int lp_info(const lp_handle* h, int64_t* info);
  * registers, above 256 points; bit 2: registers budgeted for up to 4 waves
  * per SIMD, as many as the blocks' LDS admits, instead of 2; bits 0 and 3
  * have no effect; default 14; recompiles), key 13 = slices per block of
- * lp_fwd's log-polar -> polar gather (>= 1, default 4; each block reads its
- * tile's coordinates once), key 14 = lp_fwd's image -> log-polar gather
+ * lp_fwd's log-polar -> polar gather (>= 1, default 4, halved like key 3; each
+ * block reads its tile's coordinates once), key 14 = lp_fwd's image -> log-polar gather
  * reads every tap from global memory, one thread per point (1), instead of
  * from LDS-staged tile boxes (0, the default): a measurement of the sampling
  * that a gather fused into the row pass would do.  Returns LP_ERR_ARG for bad

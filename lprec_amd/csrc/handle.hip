@@ -467,6 +467,29 @@ std::vector<lpk::GTile> tile_grid(Coord coord, const std::vector<int>& spans, in
     return out;
 }
 
+// Rows of the gather tiles over `points` output points: 64, fewer while the
+// handle's slices would give the chip less than one tile per CU (N = 64, 1
+// slice: 64 -> 8 rows, Cartesian gather 16.5 -> 8.8 us; N = 256, 4 slices:
+// 32 rows, 18 -> 14 us; wherever there are more tiles, 64 is faster).
+int tile_rows(long long points, int Ns) {
+    int tr = 64;
+    while (tr > 8 && points / (tr * 32) * Ns < 256) tr /= 2;
+    return tr;
+}
+
+// The tiles that build(rows) makes, with at least `rows` rows: more while the
+// boxes of a slice (halos grow as tiles shrink) exceed the half-spectrum
+// buffer, where the transposes stage them.
+template <class Build>
+std::vector<lpk::GTile> fit_tiles(int rows, size_t room, Build build) {
+    for (;; rows *= 2) {
+        std::vector<lpk::GTile> t = build(rows);
+        size_t total = 0;
+        for (const auto& g : t) total += (size_t)std::max(g.bw, 0) * std::max(g.bh, 0);
+        if (rows >= 64 || total <= room) return t;
+    }
+}
+
 // [lo, hi) theta columns of each (span, row) of the log-polar grids that the
 // source boxes of a gather's tiles cover; a row whose boxes wrap around the
 // periodic theta axis gets the whole row
@@ -1238,20 +1261,25 @@ int lp_init_fwd(lp_handle* h, const int32_t* pi, const float* pf) {
     std::vector<int2> rng = row_ranges(cmap, Nr, Nt);
     std::vector<lpk::GTile> tF, tP;
     try {
-        // image -> LP gather: tiles of 32 rho x 64 theta per span, kept where
+        // image -> LP gather: tiles of 64 rho x 32 theta per span, kept where
         // they meet the non-empty theta range of one of their rows
-        for (int k = 0; k < 3; ++k) {
-            auto coord = [&](int, int r, int c) { return cmap[(size_t)k * npts + (size_t)r * Nt + c]; };
-            auto keep = [&](int r0, int c0, int nr, int nc) {
-                for (int r = r0; r < r0 + nr; ++r) {
-                    int2 q = rng[(size_t)k * Nr + r];
-                    if (q.x < c0 + nc && q.y > c0) return true;
-                }
-                return false;
-            };
-            auto t = tile_grid(coord, {k}, 0, Nr, Nt, 64, 32, h->box_cap, (h->box_rule >> 0) & 1, keep, h->boxF);
-            tF.insert(tF.end(), t.begin(), t.end());
-        }
+        tF = fit_tiles(tile_rows(3LL * Nc, h->Ns), 6 * (size_t)h->h * Nr, [&](int rows) {
+            std::vector<lpk::GTile> all;
+            h->boxF = 0;
+            for (int k = 0; k < 3; ++k) {
+                auto coord = [&](int, int r, int c) { return cmap[(size_t)k * npts + (size_t)r * Nt + c]; };
+                auto keep = [&](int r0, int c0, int nr, int nc) {
+                    for (int r = r0; r < r0 + nr; ++r) {
+                        int2 q = rng[(size_t)k * Nr + r];
+                        if (q.x < c0 + nc && q.y > c0) return true;
+                    }
+                    return false;
+                };
+                auto t = tile_grid(coord, {k}, 0, Nr, Nt, rows, 32, h->box_cap, (h->box_rule >> 0) & 1, keep, h->boxF);
+                all.insert(all.end(), t.begin(), t.end());
+            }
+            return all;
+        });
         // LP -> polar gather over the kept angles (user rows), per span
         const int P0 = h->P0, lb = N / 2 - h->cor, os = h->os, N0 = h->N0;
         for (int k = 0; k < 3; ++k) {
@@ -1263,7 +1291,7 @@ int lp_init_fwd(lp_handle* h, const int32_t* pi, const float* pf) {
                 if (spanrow[(size_t)a * os] != k) return h->fail(LP_ERR_UNSUPPORTED, "span rows are not contiguous");
             auto coord = [&](int, int a, int x) { return p2lp[(size_t)a * os * N + x + lb]; };
             auto keep = [](int, int, int, int) { return true; };
-            auto t = tile_grid(coord, {k}, ab, ae, N0, 64, 32, h->box_cap, (h->box_rule >> 1) & 1, keep, h->boxP);
+            auto t = tile_grid(coord, {k}, ab, ae, N0, tile_rows((long long)P0 * N0, h->Ns), 32, h->box_cap, (h->box_rule >> 1) & 1, keep, h->boxP);
             tP.insert(tP.end(), t.begin(), t.end());
         }
     } catch (const std::exception& e) {
@@ -1409,23 +1437,32 @@ int lp_init_adj(lp_handle* h, const int32_t* pi, const float* pf) {
     std::vector<int2> rng = row_ranges(cmap, Nr, Nt);
     std::vector<lpk::GTile> tA, tC;
     try {
-        for (int k = 0; k < 3; ++k) {
-            auto coord = [&](int, int r, int c) { return cmap[(size_t)k * npts + (size_t)r * Nt + c]; };
-            auto keep = [&](int r0, int c0, int nr, int nc) {
-                for (int r = r0; r < r0 + nr; ++r) {
-                    int2 q = rng[(size_t)k * Nr + r];
-                    if (q.x < c0 + nc && q.y > c0) return true;
-                }
-                return false;
-            };
-            auto t = tile_grid(coord, {k}, 0, Nr, Nt, 64, 32, h->box_cap, (h->box_rule >> 2) & 1, keep, h->boxA);
-            tA.insert(tA.end(), t.begin(), t.end());
-        }
+        const size_t room = 6 * (size_t)h->h * Nr;
+        tA = fit_tiles(tile_rows(3LL * (Nl + Nw), h->Ns), room, [&](int rows) {
+            std::vector<lpk::GTile> all;
+            h->boxA = 0;
+            for (int k = 0; k < 3; ++k) {
+                auto coord = [&](int, int r, int c) { return cmap[(size_t)k * npts + (size_t)r * Nt + c]; };
+                auto keep = [&](int r0, int c0, int nr, int nc) {
+                    for (int r = r0; r < r0 + nr; ++r) {
+                        int2 q = rng[(size_t)k * Nr + r];
+                        if (q.x < c0 + nc && q.y > c0) return true;
+                    }
+                    return false;
+                };
+                auto t = tile_grid(coord, {k}, 0, Nr, Nt, rows, 32, h->box_cap, (h->box_rule >> 2) & 1, keep, h->boxA);
+                all.insert(all.end(), t.begin(), t.end());
+            }
+            return all;
+        });
         // LP -> Cartesian: user image tiles, the three spans of a tile consecutive
         const int o = N / 2 - h->N0 / 2;
         auto coordC = [&](int k, int y, int x) { return cmapC[(size_t)k * NN + (size_t)(y + o) * N + x + o]; };
         auto keepC = [](int, int, int, int) { return true; };
-        tC = tile_grid(coordC, {0, 1, 2}, 0, h->N0, h->N0, 64, 32, h->box_cap, (h->box_rule >> 3) & 1, keepC, h->boxC);
+        tC = fit_tiles(tile_rows((long long)h->N0 * h->N0, h->Ns), room, [&](int rows) {
+            h->boxC = 0;
+            return tile_grid(coordC, {0, 1, 2}, 0, h->N0, h->N0, rows, 32, h->box_cap, (h->box_rule >> 3) & 1, keepC, h->boxC);
+        });
     } catch (const std::exception& e) {
         return h->fail(LP_ERR_UNSUPPORTED, e.what());
     }

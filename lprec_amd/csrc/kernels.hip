@@ -1783,8 +1783,27 @@ void launch_col_iir(const float* in, float* out, int nz, int L, int W, int chunk
     }
 }
 
-void launch_gather(const Gather& g, const GTile* tiles, int ntiles, int kind, hipStream_t s) {
+// Slices per block of a tiled gather or scatter, lowered while the launch
+// would have fewer than `most` blocks: a block takes its slices in turn, so
+// few blocks leave the chip idle and more only spread the coordinate reads.
+static int fit_slices(int zgroup, int nz, long long tiles, long long most) {
+    while (zgroup > 1 && tiles * ((nz + zgroup - 1) / zgroup) < most) zgroup /= 2;
+    return zgroup;
+}
+
+// Blocks below which the slices per block are lowered, per kind.  Measured
+// with 4, 2 and 1 slices per block (us per call; N0 x slices): image -> LP
+// 39 / 30 / 27 at 512 x 8, 142 / 124 / 137 at 1024 x 16; sinogram -> LP 32 /
+// 28 / 27, 144 / 147 / 160; LP -> polar 26 / 20 / 21, 97 / 96 / 103; the
+// Cartesian gather and the scatters, which keep nothing from slice to slice,
+// 64 / 38 / 27 (adj_T 901 / 609 / 453), 160 / 142 / 135 (2863 / 2682 / 2645).
+// At 2048 x 32 all are best at 4 or level.
+constexpr long long kFitBlocks[4] = {8192, 4096, 2048, 16384}, kFitScatter = 16384;
+
+void launch_gather(const Gather& g0, const GTile* tiles, int ntiles, int kind, hipStream_t s) {
     if (ntiles <= 0) return;
+    Gather g = g0;
+    g.zgroup = fit_slices(g.zgroup, g.nz, ntiles / g.group, kFitBlocks[kind & 3]);
     dim3 grid((ntiles / g.group) * ((g.nz + g.zgroup - 1) / g.zgroup));
     // whole 64-float chunks for stage_box
     size_t lds = (size_t)((g.box_floats + 63) & ~63) * sizeof(float);
@@ -2440,6 +2459,7 @@ void launch_scatter(const Scatter& g0, const GTile* tiles, int ntiles, int kind,
     int st = std::max(1, (int)(0.618 * ng));
     while (std::gcd(st, ng) != 1) ++st;
     g.tstride = st;
+    g.zgroup = fit_slices(g.zgroup, g.nz, ng, kFitScatter);
     dim3 grid(ng * ((g.nz + g.zgroup - 1) / g.zgroup));
     size_t lds = (size_t)g.box_floats * sizeof(float);
     if (g.perm) {
