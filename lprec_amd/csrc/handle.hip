@@ -151,6 +151,8 @@ struct lp_handle {
     int2* d_inrowsA = nullptr;
     unsigned char* d_outrowsF = nullptr;  // [3][Nrho] rows the output gather reads
     unsigned char* d_outrowsA = nullptr;
+    unsigned short* d_outbitsF = nullptr;   // the same, a lane's 16 rows in one word
+    unsigned short* d_outbitsA = nullptr;
     // LDS-tiled gathers: tile lists and the largest source box of each
     lpk::GTile* d_tilesF = nullptr;   // image -> LP (per span)
     lpk::GTile* d_tilesP = nullptr;   // LP -> polar (per span)
@@ -559,6 +561,16 @@ std::vector<unsigned char> read_rows(const std::vector<int2>& wrng) {
         if (!out[i]) all = false;
     }
     if (all) out.clear();
+    return out;
+}
+
+// out_rows as the bit masks of RowPass.out_bits (Nr a multiple of 16)
+std::vector<unsigned short> row_bits(const std::vector<unsigned char>& rows, int Nr) {
+    const int T = Nr / 16;
+    std::vector<unsigned short> out(rows.empty() ? 0 : 3 * (size_t)T, 0);
+    for (size_t k = 0; k < out.size(); ++k)
+        for (int q = 0; q < 16; ++q)
+            if (rows[k / T * Nr + k % T + (size_t)q * T]) out[k] = (unsigned short)(out[k] | 1u << q);
     return out;
 }
 
@@ -1314,7 +1326,9 @@ int lp_init_fwd(lp_handle* h, const int32_t* pi, const float* pf) {
         std::vector<int2> in_rows = data_rows(rng, Nr);
         std::vector<unsigned char> out_rows = read_rows(wrng);
         if (!in_rows.empty() && (rc = h->upload(&h->d_inrowsF, in_rows))) return rc;
-        if (!out_rows.empty() && (rc = h->upload(&h->d_outrowsF, out_rows))) return rc;
+        if (!out_rows.empty() && ((rc = h->upload(&h->d_outrowsF, out_rows)) ||
+                                  (rc = h->upload(&h->d_outbitsF, row_bits(out_rows, Nr)))))
+            return rc;
     }
     if ((rc = h->upload(&h->d_cmapF, cmap)) || (rc = h->upload(&h->d_rangeF, rng)) || (rc = h->upload(&h->d_p2lp, p2lp)) ||
         (rc = h->upload(&h->d_spanrow, spanrow)) || (rc = h->upload(&h->d_fzF, fzT)) ||
@@ -1482,7 +1496,9 @@ int lp_init_adj(lp_handle* h, const int32_t* pi, const float* pf) {
         std::vector<int2> in_rows = data_rows(rng, Nr);
         std::vector<unsigned char> out_rows = read_rows(wrng);
         if (!in_rows.empty() && (rc = h->upload(&h->d_inrowsA, in_rows))) return rc;
-        if (!out_rows.empty() && (rc = h->upload(&h->d_outrowsA, out_rows))) return rc;
+        if (!out_rows.empty() && ((rc = h->upload(&h->d_outrowsA, out_rows)) ||
+                                  (rc = h->upload(&h->d_outbitsA, row_bits(out_rows, Nr)))))
+            return rc;
     }
     if ((rc = h->upload(&h->d_tilesA, tA)) || (rc = h->upload(&h->d_tilesC, tC))) return rc;
     if ((rc = stage_tables(h, tA, N, h->P, false, h->stA)) || (rc = stage_tables(h, tC, Nt, Nr, true, h->stC)))
@@ -1577,6 +1593,7 @@ static lpk::RowPass row_pass(lp_handle* h, int nz) {
     rp.fft16 = h->fft16;
     rp.in_rows = nullptr;
     rp.out_rows = nullptr;
+    rp.out_bits = nullptr;
     const bool rtc = h->rtc_mode;
     rp.rtc_rows_fwd = rtc ? h->rtc_fn[0] : nullptr;
     rp.rtc_rows_inv = rtc ? h->rtc_fn[1] : nullptr;
@@ -1616,6 +1633,7 @@ static int fwd_chain(lp_handle* h, float* R, const float* f, int ns0, hipStream_
     if (!h->stop_after) {   // (stage-wise tests read every row)
         rp.in_rows = h->d_inrowsF;
         rp.out_rows = h->d_outrowsF;
+        rp.out_bits = h->d_outbitsF;
     }
     const long long grid = (long long)h->Nr * h->Nt;
     {   // image -> log-polar samples x e^rho into F (aliases G)
@@ -1734,6 +1752,7 @@ int lp_adj(lp_handle* h, float* f, const float* R, int ns0, void* stream) {
     if (!h->stop_after) {   // (stage-wise tests read every row)
         rp.in_rows = h->d_inrowsA;
         rp.out_rows = h->d_outrowsA;
+        rp.out_bits = h->d_outbitsA;
     }
     lpk::Src src{h->d_Rc, N, h->P, (long long)h->P * N};
     const long long grid = (long long)h->Nr * h->Nt;

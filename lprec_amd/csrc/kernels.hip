@@ -98,7 +98,7 @@ __device__ __forceinline__ void st_at(T* base, unsigned off, T v) {
 // global_load_lds with the hint, kCpolNT, and S out): 1.26 / 1.28 against
 // 1.33 / 1.35 ms, neither half alone faster; on the radix-16 inverse row
 // pass at h = 512: 0.167 / 0.135 against 0.177 / 0.141 ms.  Slower on the
-// forward row pass (F reads, S writes); no gain on k_cols16.
+// forward row pass (F reads, S writes); no gain on shorter columns.
 constexpr int kCpolNT = 2;   // cache-policy operand of the load-to-LDS builtin: nt
 typedef float v2f_nt __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float2 ld_at_nt(const float2* base, unsigned off) {
@@ -825,6 +825,23 @@ __global__ void k_rows_inv(RowPass rp, float* __restrict__ G, const int2* __rest
 // FFT.  Column 0 carries the theta-DC and theta-Nyquist columns packed as
 // X0 + i Xh; they are separated by Hermitian symmetry, multiplied by their own
 // spectra and re-packed.
+// The product of frequency 0: column pair X0 + i Xh in smc, separated, multiplied
+// by the kernel columns of the two frequencies and packed again.
+__device__ __forceinline__ void product_dc(float2* smc, int M, const float2* __restrict__ fz,
+                                           const float2* __restrict__ fzh, int conj) {
+    for (int k = threadIdx.x; k <= M / 2; k += blockDim.x) {
+        int km = k == 0 ? 0 : M - k;
+        float2 A = smc[lidx(k)], Bc = cconj(smc[lidx(km)]);
+        float2 D = make_float2(0.5f * (A.x + Bc.x), 0.5f * (A.y + Bc.y));
+        float2 E = make_float2(0.5f * (A.x - Bc.x), 0.5f * (A.y - Bc.y));
+        float2 Q = make_float2(E.y, -E.x);  // E / i
+        float2 yk = cadd(cmul(D, fzval(fz, k, conj)), rot90(cmul(Q, fzval(fzh, k, conj)), 1));
+        float2 ykm = cadd(cmul(cconj(D), fzval(fz, km, conj)), rot90(cmul(cconj(Q), fzval(fzh, km, conj)), 1));
+        smc[lidx(k)] = yk;
+        if (km != k) smc[lidx(km)] = ykm;
+    }
+}
+
 template <int EPT>
 __global__ void k_cols(RowPass rp, FftPlan planM, const float2* __restrict__ twM, const float2* __restrict__ fzT) {
     extern __shared__ float2 smc[];
@@ -843,17 +860,7 @@ __global__ void k_cols(RowPass rp, FftPlan planM, const float2* __restrict__ twM
         __syncthreads();
         fft_lds<EPT>(smc, M, 1, planM, twM, -1);
         if (f == 0) {
-            for (int k = threadIdx.x; k <= M / 2; k += blockDim.x) {
-                int km = k == 0 ? 0 : M - k;
-                float2 A = smc[lidx(k)], Bc = cconj(smc[lidx(km)]);
-                float2 D = make_float2(0.5f * (A.x + Bc.x), 0.5f * (A.y + Bc.y));
-                float2 E = make_float2(0.5f * (A.x - Bc.x), 0.5f * (A.y - Bc.y));
-                float2 Q = make_float2(E.y, -E.x);  // E / i
-                float2 yk = cadd(cmul(D, fzval(fz, k, rp.conj)), rot90(cmul(Q, fzval(fzh, k, rp.conj)), 1));
-                float2 ykm = cadd(cmul(cconj(D), fzval(fz, km, rp.conj)), rot90(cmul(cconj(Q), fzval(fzh, km, rp.conj)), 1));
-                smc[lidx(k)] = yk;
-                if (km != k) smc[lidx(km)] = ykm;
-            }
+            product_dc(smc, M, fz, fzh, rp.conj);
         } else {
             for (int i = threadIdx.x; i < M; i += blockDim.x) smc[lidx(i)] = cmul(smc[lidx(i)], fzval(fz, i, rp.conj));
         }
@@ -888,130 +895,6 @@ __device__ __forceinline__ void twiddle16(float2* v, const float2* __restrict__ 
     v[13] = cmul(v[13], cmul(w1, w12));
     v[14] = cmul(v[14], cmul(w2, w12));
     v[15] = cmul(v[15], cmul(w3, w12));
-}
-
-// Column pass for power-of-two M = 16 * MID * 16 (MID in 1, 2, 4, 8, 16):
-// M/16 threads per column hold one radix-16 butterfly each.  Stage 0 reads
-// HBM directly, the last forward stage leaves thread i holding outputs
-// i + q M/16 -- exactly the inputs of the first inverse stage -- so the
-// kernel-spectrum multiply and the inverse start in registers; 4 LDS
-// exchanges in total.  C columns share a 256-thread block for small M.
-template <int MID>
-__device__ __forceinline__ void col_mid_stage(float2* buf, int M, int dir, const float2* __restrict__ tw, int li,
-                                              bool worker) {
-    // radix-MID stage, Ns = 16; thread li handles 16/MID butterflies
-    constexpr int NB = 16 / MID;
-    const int nbf = M / MID;
-    float2 v[NB][MID];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        int j = li * NB + b;
-#pragma unroll
-        for (int q = 0; q < MID; ++q) v[b][q] = buf[lidx(j + q * nbf)];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        int j = li * NB + b;
-        int k = j & 15;
-        const int tstep = M / (16 * MID);
-        if (MID == 16) {
-            twiddle16(v[b], tw, k * tstep, dir);   // powers formed as they are applied
-        } else if (MID > 1) {
-            float2 w[MID > 1 ? MID : 2];
-            twiddle_pows<MID>(tw, k * tstep, dir, w);
-#pragma unroll
-            for (int q = 1; q < MID; ++q) v[b][q] = cmul(v[b][q], w[q]);
-        }
-        if (MID == 16) dft16(v[b], dir);
-        else if (MID == 8) dft_small<8>(v[b], dir);
-        else if (MID == 4) dft_small<4>(v[b], dir);
-        else if (MID == 2) dft_small<2>(v[b], dir);
-        int dst = (j - k) * MID + k;
-        if (worker) {
-#pragma unroll
-            for (int q = 0; q < MID; ++q) buf[lidx(dst + q * 16)] = v[b][q];
-        }
-    }
-    __syncthreads();
-}
-
-
-template <int MID>
-__global__ void __launch_bounds__(256, 2) k_cols16(RowPass rp, const float2* __restrict__ twM,
-                                                   const float2* __restrict__ fzT) {
-    extern __shared__ float2 smc[];
-    // one column per block; block-uniform base pointers with 32-bit lane
-    // offsets keep the 16 addresses out of the vector registers
-    constexpr int M = 256 * MID;            // == rp.Nrho (checked on launch)
-    constexpr int T16 = M / 16;             // working threads per column
-    const int h = rp.h;
-    const int li = min((int)threadIdx.x, T16 - 1);
-    const bool worker = (int)threadIdx.x < T16;
-    // logical order: slice groups, then spans of one column are neighbours
-    // (they read the same kernel-spectrum column); column 0 runs on k_cols
-    const int nzg = (rp.nz + rp.zgroup - 1) / rp.zgroup;
-    const int lb = xcd_block(blockIdx.x, gridDim.x);
-    const int zg = lb % nzg, t = lb / nzg;
-    const int span = t % 3, f = 1 + t / 3;
-    float2* buf = smc;
-    const float2* fz = fzT + (size_t)f * M;
-    const int z0 = zg * rp.zgroup;
-    const int z1 = min(z0 + rp.zgroup, rp.nz);
-    constexpr int tstep3 = M / (16 * MID * 16);  // last stage: Ns = 16 MID, radix 16 (= 1)
-    const int2 ir = rp.in_rows ? rp.in_rows[span] : make_int2(0, M);
-    unsigned smask = 0xffffu;   // stored rows among li + q T16, read once
-    if (rp.out_rows) {
-        const unsigned char* om = rp.out_rows + (size_t)span * M;
-        smask = 0;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) smask |= om[li + q * T16] ? (1u << q) : 0u;
-    }
-    for (int z = z0; z < z1; ++z) {
-        float2* col = rp.S + (((size_t)span * rp.nz + z) * h + f) * (size_t)M;
-        float2 v[16];
-        // ---- forward stage 0: radix 16, Ns = 1, straight from HBM (rows
-        // without data are zeros)
-#pragma unroll
-        for (int q = 0; q < 16; ++q) {
-            const int i = li + q * T16;
-            v[q] = (i >= ir.x && i < ir.y) ? col[i] : make_float2(0.f, 0.f);
-        }
-        dft16(v, -1);
-        if (worker) {
-#pragma unroll
-            for (int q = 0; q < 16; ++q) buf[lidx(li * 16 + q)] = v[q];
-        }
-        __syncthreads();
-        if (MID > 1) col_mid_stage<MID>(buf, M, -1, twM, li, worker);
-        // ---- forward last stage: radix 16, Ns = M/16, k = li
-#pragma unroll
-        for (int q = 0; q < 16; ++q) v[q] = buf[lidx(li + q * T16)];
-        twiddle16(v, twM, li * tstep3, -1);
-        dft16(v, -1);
-        // v[q] = spectrum at kappa = li + q M/16: kernel multiply in registers
-#pragma unroll
-        for (int q = 0; q < 16; ++q) v[q] = cmul(v[q], fzval(fz, li + q * T16, rp.conj));
-        // ---- inverse stage 0 (radix 16, Ns = 1)
-        dft16(v, +1);
-        __syncthreads();
-        if (worker) {
-#pragma unroll
-            for (int q = 0; q < 16; ++q) buf[lidx(li * 16 + q)] = v[q];
-        }
-        __syncthreads();
-        if (MID > 1) col_mid_stage<MID>(buf, M, +1, twM, li, worker);
-#pragma unroll
-        for (int q = 0; q < 16; ++q) v[q] = buf[lidx(li + q * T16)];
-        twiddle16(v, twM, li * tstep3, +1);
-        dft16(v, +1);
-        if (worker) {
-#pragma unroll
-            for (int q = 0; q < 16; ++q)
-                if (smask & (1u << q)) col[li + q * T16] = v[q];
-        }
-        __syncthreads();
-    }
 }
 
 // Block barrier that waits only for this wave's LDS traffic (lgkmcnt), not
@@ -1049,116 +932,189 @@ __device__ __forceinline__ void twiddle16_w(float2* v, const float2* w, int dir)
     v[15] = cmul(v[15], cmul(w3, w12));
 }
 
-// Column pass for M = 4096 (16 x 16 x 16) with the next slice's column
-// streamed from HBM into LDS (load-to-LDS, no registers) while the current one
-// is transformed.  The twiddles and the kernel-spectrum column are loaded once
-// per block, so no other global load shares the vector-memory counter with the
-// stream and every barrier inside a slice waits for LDS traffic only.
-__global__ void __launch_bounds__(256, 2) k_cols4096(RowPass rp, const float2* __restrict__ twM,
-                                                     const float2* __restrict__ fzT) {
-    constexpr int M = 4096, T16 = 256;
-    __shared__ float2 buf[lds_slots(M)];
-    __shared__ __align__(16) float2 pre[M];
+// 16 bytes per lane straight to LDS (lane l of the wave at dst + 2 l).  (A
+// function of its own: the host pass drops a kernel template that names the
+// builtin in a lambda.)
+template <bool kNT>
+__device__ __forceinline__ void load_lds16(const float2* src, float2* dst) {
+    __builtin_amdgcn_global_load_lds(src, dst, 16, 0, kNT ? kCpolNT : 0);
+}
+
+// Column pass for power-of-two M = 256 MID (MID in 1, 2, 4, 8, 16): FFT along
+// rho of the columns of one theta frequency, kernel spectrum, inverse FFT, one
+// radix-16 butterfly per lane and stage (16 x MID x 16), M / 16 lanes per
+// column; short columns share a wave (C adjacent frequencies).  A block takes
+// `items` of the 3 nz columns (span, slice) of its frequencies in turn and
+// streams the next one from HBM into LDS (load-to-LDS, no registers) while
+// the current one is transformed: twiddles and the kernel-spectrum column are
+// loaded once per block, so no other global load shares the vector-memory
+// counter with the stream and every barrier inside a column waits for LDS
+// traffic only.  The last forward stage leaves lane li holding outputs
+// li + q M / 16, the inputs of the first inverse stage, so the product and the
+// turn happen in registers; 4 LDS exchanges in total.
+// Frequency 0 carries the theta-DC and -Nyquist columns packed as X0 + i Xh:
+// with B the output at M - kappa, (A + conj B) / 2 and (A - conj B) / 2i are
+// their spectra, multiplied by their own kernel columns and packed again.
+// (As a launch of its own this one column took 16-42 us of every call before
+// the others could start: the pass 28 -> 13 us at N = 512, 1 slice.  As
+// blocks of their own with the mixed-radix FFT they bound the launch: 24 us.)
+// At M = 4096 the stream runs at the copy rate: 1.23 ms per 32 slices (1.25
+// with the separate launch); M = 2048, 16 slices 234 -> 185 us.
+template <int MID>
+struct ColShape {
+    static constexpr int M = 256 * MID, T16 = 16 * MID, C = T16 >= 64 ? 1 : 64 / T16, NT = C * T16;
+};
+
+template <int MID>
+__global__ void __launch_bounds__(ColShape<MID>::NT, 2) k_cols_stream(RowPass rp, int items,
+                                                                      const float2* __restrict__ twM,
+                                                                      const float2* __restrict__ fzT) {
+    constexpr int M = ColShape<MID>::M, T16 = ColShape<MID>::T16, C = ColShape<MID>::C, NT = ColShape<MID>::NT;
+    constexpr int NB = 16 / MID, nbf = 256, LW = MID == 16 ? 4 : MID == 8 ? 3 : MID == 4 ? 2 : 1;
+    constexpr bool kNT = MID == 16;   // the non-temporal hints (no gain at shorter columns)
+    __shared__ float2 buf_s[C * lds_slots(M)];
+    __shared__ __align__(16) float2 pre_s[C * M];
     const int h = rp.h;
-    const int li = threadIdx.x;
-    const int nzg = (rp.nz + rp.zgroup - 1) / rp.zgroup;
+    const int li = threadIdx.x % T16, cl = threadIdx.x / T16;
+    float2* buf = buf_s + cl * lds_slots(M);
+    const float2* pre = pre_s + cl * M;
+    // logical order: the item groups of one frequency are neighbours (they
+    // read the same kernel-spectrum column)
+    const int ng = (3 * rp.nz + items - 1) / items;
     const int lb = xcd_block(blockIdx.x, gridDim.x);
-    const int zg = lb % nzg, t = lb / nzg;
-    const int span = t % 3, f = 1 + t / 3;
-    const int z0 = zg * rp.zgroup;
-    const int z1 = min(z0 + rp.zgroup, rp.nz);
-    const int wv = li >> 6, ln = li & 63;
-    // 128-row chunks of the column that carry data (a multiple of 128 bounds
-    // the rows with data); the others stay zero in `pre`
-    const int2 ir = rp.in_rows ? rp.in_rows[span] : make_int2(0, M);
-    const int c_lo = ir.x >> 7, c_hi = (ir.y + 127) >> 7;
-    // rows of this thread's 16 outputs (li + q 256) that are stored: read once,
-    // before the stream starts, so that no other global load joins it
-    unsigned smask = 0xffffu;
-    if (rp.out_rows) {
-        const unsigned char* om = rp.out_rows + (size_t)span * M;
-        smask = 0;
+    const int f0 = lb / ng * C, f = f0 + cl;
+    const int i0 = (lb % ng) * items, i1 = min(i0 + items, 3 * rp.nz);
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), ln = threadIdx.x & 63;
+    // (S is [3][nz]: column `it` of a frequency is it h M values further on)
+    auto column = [&](int it, int fr) { return rp.S + ((size_t)it * h + fr) * (size_t)M; };
+    // 128-row chunks outside the rows that carry data are zeros
+    auto prefetch = [&](int it, int span) {
+        const int2 ir = rp.in_rows ? rp.in_rows[span] : make_int2(0, M);
+        const int c_lo = ir.x >> 7, c_hi = (ir.y + 127) >> 7;
 #pragma unroll
-        for (int q = 0; q < 16; ++q) smask |= om[li + q * T16] ? (1u << q) : 0u;
-    }
-    for (int i = li; i < M; i += T16)
-        if ((i >> 7) < c_lo || (i >> 7) >= c_hi) pre[i] = make_float2(0.f, 0.f);
-    auto prefetch = [&](int z) {
-        const float2* col = rp.S + (((size_t)span * rp.nz + z) * h + f) * (size_t)M;
-#pragma unroll
-        for (int c = 0; c < M / 128 / 4; ++c) {
-            const int cc = wv + 4 * c;
-            if (cc >= c_lo && cc < c_hi)
-                __builtin_amdgcn_global_load_lds(col + cc * 128 + ln * 2, pre + cc * 128, 16, 0, kCpolNT);
+        for (int c0 = 0; c0 < C * M / 128; c0 += NT / 64) {
+            const int cc = c0 + wv, col = cc / (M / 128), ch = cc - col * (M / 128);   // uniform over the wave
+            float2* dst = pre_s + cc * 128;
+            if (ch >= c_lo && ch < c_hi)
+                load_lds16<kNT>(column(it, f0 + col) + ch * 128 + ln * 2, dst);
+            else
+                *reinterpret_cast<float4*>(dst + ln * 2) = make_float4(0.f, 0.f, 0.f, 0.f);
         }
     };
-    prefetch(z0);
-    // per-block constants: middle-stage twiddles (k = li & 15, step 16),
-    // last-stage twiddles (k = li, step 1), the kernel-spectrum column
-    float2 wm[4], wl[4], kz[16];
-    {
-        const int km = (li & 15) * 16;
-        wm[0] = twM[km]; wm[1] = twM[2 * km]; wm[2] = twM[4 * km]; wm[3] = twM[8 * km];
-        wl[0] = twM[li]; wl[1] = twM[2 * li]; wl[2] = twM[4 * li]; wl[3] = twM[8 * li];
-        const float2* fz = fzT + (size_t)f * M;
+    int span = __builtin_amdgcn_readfirstlane(i0 / rp.nz), left = (span + 1) * rp.nz - i0;   // columns left in the span
+    prefetch(i0, span);
+    // per-block constants: middle-stage twiddles (k = j & 15 of butterfly j),
+    // last-stage twiddles (k = li), the kernel-spectrum column, the stored
+    // rows among li + q M / 16 of each span
+    float2 wm[NB][LW], wl[4], kz[16];
 #pragma unroll
-        for (int q = 0; q < 16; ++q) kz[q] = fzval(fz, li + q * T16, rp.conj);
-    }
-    for (int z = z0; z < z1; ++z) {
-        float2* col = rp.S + (((size_t)span * rp.nz + z) * h + f) * (size_t)M;
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int l = 0; l < LW; ++l) wm[b][l] = twM[(((li * NB + b) & 15) * (M / (16 * MID))) << l];
+#pragma unroll
+    for (int l = 0; l < 4; ++l) wl[l] = twM[(li * (M / (256 * MID))) << l];
+    const float2* fz = fzT + (size_t)f * M;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) kz[q] = fzval(fz, li + q * T16, rp.conj);
+    unsigned smask[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) smask[k] = rp.out_bits ? rp.out_bits[k * T16 + li] : 0xffffu;
+    auto mid_stage = [&](int dir) {
+        if constexpr (MID > 1) {
+            float2 u[NB][MID];
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int q = 0; q < MID; ++q) u[b][q] = buf[lidx(li * NB + b + q * nbf)];
+            lds_barrier();
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const int j = li * NB + b, k = j & 15;
+                if constexpr (MID == 16) {
+                    twiddle16_w(u[b], wm[b], dir);
+                } else {
+                    float2 w[MID];
+#pragma unroll
+                    for (int q = 1; q < MID; ++q) {
+                        if ((q & (q - 1)) == 0) w[q] = dir > 0 ? cconj(wm[b][q == 1 ? 0 : q == 2 ? 1 : 2]) : wm[b][q == 1 ? 0 : q == 2 ? 1 : 2];
+                        else w[q] = cmul(w[q & (q - 1)], w[q & -q]);
+                        u[b][q] = cmul(u[b][q], w[q]);
+                    }
+                }
+                if constexpr (MID == 16) dft16(u[b], dir);
+                else dft_small<MID>(u[b], dir);
+                const int dst = (j - k) * MID + k;
+#pragma unroll
+                for (int q = 0; q < MID; ++q) buf[lidx(dst + q * 16)] = u[b][q];
+            }
+            lds_barrier();
+        }
+    };
+    for (int it = i0; it < i1; ++it) {
         float2 v[16];
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();   // column z is in pre
+        __syncthreads();   // column `it` is in pre
 #pragma unroll
         for (int q = 0; q < 16; ++q) v[q] = pre[li + q * T16];
         dft16(v, -1);
 #pragma unroll
         for (int q = 0; q < 16; ++q) buf[lidx(li * 16 + q)] = v[q];
         lds_barrier();   // pre has been read by every wave
-        if (z + 1 < z1) prefetch(z + 1);
-        // middle stage (radix 16, Ns = 16)
-        {
-            const int j = li, k = j & 15;
-#pragma unroll
-            for (int q = 0; q < 16; ++q) v[q] = buf[lidx(j + q * 256)];
-            lds_barrier();
-            twiddle16_w(v, wm, -1);
-            dft16(v, -1);
-            const int dst = (j - k) * 16 + k;
-#pragma unroll
-            for (int q = 0; q < 16; ++q) buf[lidx(dst + q * 16)] = v[q];
-            lds_barrier();
-        }
+        if (it + 1 < i1) prefetch(it + 1, span + (left == 1));
+        mid_stage(-1);
 #pragma unroll
         for (int q = 0; q < 16; ++q) v[q] = buf[lidx(li + q * T16)];
         twiddle16_w(v, wl, -1);
         dft16(v, -1);
+        if (f0 == 0) {   // uniform over the block
+            lds_barrier();
 #pragma unroll
-        for (int q = 0; q < 16; ++q) v[q] = cmul(v[q], kz[q]);
+            for (int q = 0; q < 16; ++q) buf[lidx(li + q * T16)] = v[q];
+            lds_barrier();
+            const float2* fzh = fzT + (size_t)h * M;
+            int lz = li;   // opaque: this branch's addresses are not held in registers for the others
+            asm volatile("" : "+v"(lz));
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int k = lz + q * T16;
+                const float2 A = v[q], Bc = cconj(buf[lidx(k == 0 ? 0 : M - k)]);
+                const float2 D = make_float2(0.5f * (A.x + Bc.x), 0.5f * (A.y + Bc.y));
+                const float2 Q = make_float2(0.5f * (A.y - Bc.y), -0.5f * (A.x - Bc.x));
+                const float2 y = cadd(cmul(D, kz[q]), rot90(cmul(Q, fzval(fzh, k, rp.conj)), 1));
+                const float2 p = cmul(A, kz[q]);
+                v[q] = f == 0 ? y : p;
+                // four outputs' operands at a time: a spill's reloads would
+                // join the vector-memory counter of the stream
+                if (q % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) v[q] = cmul(v[q], kz[q]);
+        }
         dft16(v, +1);
         lds_barrier();
 #pragma unroll
         for (int q = 0; q < 16; ++q) buf[lidx(li * 16 + q)] = v[q];
         lds_barrier();
-        {
-            const int j = li, k = j & 15;
-#pragma unroll
-            for (int q = 0; q < 16; ++q) v[q] = buf[lidx(j + q * 256)];
-            lds_barrier();
-            twiddle16_w(v, wm, +1);
-            dft16(v, +1);
-            const int dst = (j - k) * 16 + k;
-#pragma unroll
-            for (int q = 0; q < 16; ++q) buf[lidx(dst + q * 16)] = v[q];
-            lds_barrier();
-        }
+        mid_stage(+1);
 #pragma unroll
         for (int q = 0; q < 16; ++q) v[q] = buf[lidx(li + q * T16)];
         twiddle16_w(v, wl, +1);
         dft16(v, +1);
+        const unsigned sm = span == 0 ? smask[0] : span == 1 ? smask[1] : smask[2];
+        float2* col = column(it, f0);
+        unsigned lane = (unsigned)(cl * M + li) * 8u;
+        asm volatile("" : "+v"(lane));   // the 16 offsets are formed here, not held across the columns
 #pragma unroll
         for (int q = 0; q < 16; ++q)
-            if (smask & (1u << q)) st_at_nt(col, (unsigned)(li + q * T16) * 8u, v[q]);
+            if (sm & (1u << q)) {
+                if constexpr (kNT) st_at_nt(col, lane + (unsigned)(q * T16) * 8u, v[q]);
+                else st_at(col, lane + (unsigned)(q * T16) * 8u, v[q]);
+            }
+        if (--left == 0) {
+            ++span;
+            left = rp.nz;
+        }
         lds_barrier();
     }
 }
@@ -1954,34 +1910,31 @@ static int cols16_mid(int M) {
     return M / 256;
 }
 
+template <int MID>
+static void cols_stream(const RowPass& rp, const float2* twM, const float2* fzT, hipStream_t s) {
+    constexpr int C = ColShape<MID>::C;
+    // columns per block: the zgroup slices of the three spans at M = 4096
+    // (24 and 12: 1.23 / 1.21 and 1.24 / 1.19 ms per 32 slices, 6: 1.26 /
+    // 1.21), at most 6 of the shorter ones (M = 2048, 16 slices: 24 206 us,
+    // 12 203, 6 185, 3 200), fewer while the launch has less than 2048 blocks
+    int items = std::min(MID == 16 ? 3 * rp.zgroup : std::min(3 * rp.zgroup, 6), 3 * rp.nz);
+    while (items > 1 && (long long)(rp.h / C) * ((3 * rp.nz + items - 1) / items) < 2048) items = (items + 1) / 2;
+    hipLaunchKernelGGL(k_cols_stream<MID>, dim3((rp.h / C) * ((3 * rp.nz + items - 1) / items)),
+                       dim3(ColShape<MID>::NT), 0, s, rp, items, twM, fzT);
+}
+
 void launch_cols(const RowPass& rp0, const FftPlan& planM, const float2* twM, const float2* fzT, hipStream_t s) {
-    const RowPass rp = fit_zgroup(rp0, 3LL * rp0.h);
-    if (int mid = rp.fft16 ? cols16_mid(rp.Nrho) : 0) {
-        const int T16 = rp.Nrho / 16;
-        // column 0 (packed theta-DC / Nyquist pair) on the generic kernel, one
-        // block per span and slice (a few blocks only: latency-bound)
-        {
-            RowPass r0 = rp;
-            r0.zgroup = 1;
-            int nt = threads_for(rp.Nrho);
-            int ept = ept_for(rp.Nrho, nt);
-            dim3 g0(1, 3, rp.nz);
-            LP_DISPATCH_EPT(ept, k_cols, g0, dim3(nt), cols_lds_bytes(rp.Nrho), s, r0, planM, twM, fzT);
-        }
-        dim3 grid((rp.h - 1) * 3 * ((rp.nz + rp.zgroup - 1) / rp.zgroup));
-        dim3 block(std::max(T16, 64));
-        size_t lds = (size_t)lds_slots(rp.Nrho) * sizeof(float2);
-        if (rp.h > 1) {
-            switch (mid) {
-                case 1: hipLaunchKernelGGL(k_cols16<1>, grid, block, lds, s, rp, twM, fzT); break;
-                case 2: hipLaunchKernelGGL(k_cols16<2>, grid, block, lds, s, rp, twM, fzT); break;
-                case 4: hipLaunchKernelGGL(k_cols16<4>, grid, block, lds, s, rp, twM, fzT); break;
-                case 8: hipLaunchKernelGGL(k_cols16<8>, grid, block, lds, s, rp, twM, fzT); break;
-                default: hipLaunchKernelGGL(k_cols4096, grid, block, 0, s, rp, twM, fzT); break;   // static LDS
-            }
+    if (int mid = rp0.fft16 ? cols16_mid(rp0.Nrho) : 0) {
+        switch (mid) {
+            case 1: cols_stream<1>(rp0, twM, fzT, s); break;
+            case 2: cols_stream<2>(rp0, twM, fzT, s); break;
+            case 4: cols_stream<4>(rp0, twM, fzT, s); break;
+            case 8: cols_stream<8>(rp0, twM, fzT, s); break;
+            default: cols_stream<16>(rp0, twM, fzT, s); break;
         }
         return;
     }
+    const RowPass rp = fit_zgroup(rp0, 3LL * rp0.h);
     dim3 grid(rp.h, 3, (rp.nz + rp.zgroup - 1) / rp.zgroup);
     if (rp.rtc_cols) {
         RowPass rc = rp;

@@ -115,6 +115,9 @@ struct RowPass {
     // the inverse row pass skips blocks with none.
     const int2* in_rows;
     const unsigned char* out_rows;
+    // out_rows for the column pass at Nrho = 256 MID: bit q of
+    // out_bits[span * Nrho / 16 + i] is row i + q Nrho / 16
+    const unsigned short* out_bits;
     // Row and column passes compiled at run time for this handle's lengths
     // (hipFunction_t of rtc_kernels.hpp; null: the mixed-radix kernels run):
     // rows_fwd / rows_inv with rtc_R rows and rtc_rows_nt threads per block,
