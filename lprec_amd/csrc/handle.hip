@@ -134,6 +134,9 @@ struct lp_handle {
     // colour-sorted points of the tile lists (atomics-free scatters)
     unsigned short *d_permF = nullptr, *d_permP = nullptr, *d_permA = nullptr, *d_permC = nullptr;
     int *d_clsF = nullptr, *d_clsP = nullptr, *d_clsA = nullptr, *d_clsC = nullptr;
+    // tile groups with a tile that has no colouring
+    int *d_plainF = nullptr, *d_plainP = nullptr, *d_plainA = nullptr, *d_plainC = nullptr;
+    int nplainF = 0, nplainP = 0, nplainA = 0, nplainC = 0;
     // separable transpose of the polar gather (pt_ok false: the geometry does not allow it)
     int* d_pt_abeg = nullptr;
     float* d_pt_cxa = nullptr;
@@ -408,9 +411,11 @@ void colour_tile(lpk::GTile& t, Coord coord) {
 // Colours every tile of a list (threads over tiles) and lays out the
 // colour-sorted point lists: perm (r * nc + c of the points with a sample,
 // stable within a class) and the class bounds cls, both concatenated over the
-// tiles (GTile.pbase / cbase); uploaded to *d_perm / *d_cls.
+// tiles (GTile.pbase / cbase); uploaded to *d_perm / *d_cls.  The groups of
+// `group` tiles that hold an uncoloured one are listed in *d_plain.
 template <class Coord>
-int colour_list(lp_handle* h, std::vector<lpk::GTile>& tiles, Coord coord, unsigned short** d_perm, int** d_cls) {
+int colour_list(lp_handle* h, std::vector<lpk::GTile>& tiles, Coord coord, int group, unsigned short** d_perm,
+                int** d_cls, int** d_plain, int* nplain) {
     const unsigned nth = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
     std::vector<std::vector<unsigned short>> perms(tiles.size());
     std::vector<std::vector<int>> clss(tiles.size());
@@ -449,8 +454,13 @@ int colour_list(lp_handle* h, std::vector<lpk::GTile>& tiles, Coord coord, unsig
         perm.insert(perm.end(), perms[i].begin(), perms[i].end());
         cls.insert(cls.end(), clss[i].begin(), clss[i].end());
     }
+    std::vector<int> plain;
+    for (size_t i = 0; i < tiles.size(); ++i)
+        if (tiles[i].bw > 0 && tiles[i].cr == 0 && (plain.empty() || plain.back() != (int)i / group))
+            plain.push_back((int)i / group);
+    *nplain = (int)plain.size();
     int rc;
-    if ((rc = h->upload(d_perm, perm)) || (rc = h->upload(d_cls, cls))) return rc;
+    if ((rc = h->upload(d_perm, perm)) || (rc = h->upload(d_cls, cls)) || (rc = h->upload(d_plain, plain))) return rc;
     return LP_OK;
 }
 
@@ -1316,8 +1326,8 @@ int lp_init_fwd(lp_handle* h, const int32_t* pi, const float* pf) {
         const int lbp = N / 2 - h->cor, osp = h->os;
         auto coordF = [&](int k, int r, int c) { return cmap[(size_t)k * npts + (size_t)r * Nt + c]; };
         auto coordP = [&](int, int a, int x) { return p2lp[(size_t)a * osp * N + x + lbp]; };
-        if ((rc = colour_list(h, tF, coordF, &h->d_permF, &h->d_clsF)) ||
-            (rc = colour_list(h, tP, coordP, &h->d_permP, &h->d_clsP)))
+        if ((rc = colour_list(h, tF, coordF, 1, &h->d_permF, &h->d_clsF, &h->d_plainF, &h->nplainF)) ||
+            (rc = colour_list(h, tP, coordP, 1, &h->d_permP, &h->d_clsP, &h->d_plainP, &h->nplainP)))
             return rc;
     }
     if ((rc = h->upload(&h->d_tilesF, tF)) || (rc = h->upload(&h->d_tilesP, tP))) return rc;
@@ -1487,8 +1497,8 @@ int lp_init_adj(lp_handle* h, const int32_t* pi, const float* pf) {
         const int o = N / 2 - h->N0 / 2;
         auto coordA = [&](int k, int r, int c) { return cmap[(size_t)k * npts + (size_t)r * Nt + c]; };
         auto coordC = [&](int k, int y, int x) { return cmapC[(size_t)k * NN + (size_t)(y + o) * N + x + o]; };
-        if ((rc = colour_list(h, tA, coordA, &h->d_permA, &h->d_clsA)) ||
-            (rc = colour_list(h, tC, coordC, &h->d_permC, &h->d_clsC)))
+        if ((rc = colour_list(h, tA, coordA, 1, &h->d_permA, &h->d_clsA, &h->d_plainA, &h->nplainA)) ||
+            (rc = colour_list(h, tC, coordC, 3, &h->d_permC, &h->d_clsC, &h->d_plainC, &h->nplainC)))
             return rc;
     }
     if ((rc = h->upload(&h->d_wrangeA, wrng))) return rc;
@@ -1826,7 +1836,7 @@ int lp_fwd_T(lp_handle* h, float* f, const float* R, int ns0, void* stream) {
         g.scale = nullptr; g.s_row = 0;
         g.val = R; g.v_z = (long long)h->P0 * h->N0; g.v_span = 0; g.v_row = h->N0;
         g.nz = ns0; g.zgroup = h->gzgroup; g.group = 1; g.cubic = h->cubic; g.box_floats = h->boxP;
-        g.perm = h->d_permP; g.cls = h->d_clsP;
+        g.perm = h->d_permP; g.cls = h->d_clsP; g.plain = h->d_plainP; g.nplain = h->nplainP;
         lpk::launch_scatter(g, h->d_tilesP, h->ntilesP, 2, s);
     }
     lpk::RowPass rp = row_pass(h, ns0);
@@ -1843,7 +1853,7 @@ int lp_fwd_T(lp_handle* h, float* f, const float* R, int ns0, void* stream) {
         g.scale = h->d_erho; g.s_row = h->Nt;
         g.val = h->d_G; g.v_z = grid; g.v_span = (long long)ns0 * grid; g.v_row = h->Nt;
         g.nz = ns0; g.zgroup = h->gzgroup; g.group = 1; g.cubic = h->cubic; g.box_floats = h->boxF;
-        g.perm = h->d_permF; g.cls = h->d_clsF;
+        g.perm = h->d_permF; g.cls = h->d_clsF; g.plain = h->d_plainF; g.nplain = h->nplainF;
         scatter_to(h, g, h->d_tilesF, h->ntilesF, 0, h->stF, (size_t)ns0 * N * N, s);
     }
     if (h->cubic) {
@@ -1874,7 +1884,7 @@ int lp_adj_T(lp_handle* h, float* R, const float* f, int ns0, void* stream) {
         g.scale = nullptr; g.s_row = 0;
         g.val = f; g.v_z = (long long)h->N0 * h->N0; g.v_span = 0; g.v_row = h->N0;
         g.nz = ns0; g.zgroup = h->gzgroup; g.group = 3; g.cubic = h->cubic; g.box_floats = h->boxC;
-        g.perm = h->d_permC; g.cls = h->d_clsC;
+        g.perm = h->d_permC; g.cls = h->d_clsC; g.plain = h->d_plainC; g.nplain = h->nplainC;
         scatter_to(h, g, h->d_tilesC, h->ntilesC, 3, h->stC, 3 * (size_t)ns0 * grid, s);
     }
     lpk::RowPass rp = row_pass(h, ns0);
@@ -1891,7 +1901,7 @@ int lp_adj_T(lp_handle* h, float* R, const float* f, int ns0, void* stream) {
         g.scale = nullptr; g.s_row = 0;
         g.val = h->d_G; g.v_z = grid; g.v_span = (long long)ns0 * grid; g.v_row = h->Nt;
         g.nz = ns0; g.zgroup = h->gzgroup; g.group = 1; g.cubic = h->cubic; g.box_floats = h->boxA;
-        g.perm = h->d_permA; g.cls = h->d_clsA;
+        g.perm = h->d_permA; g.cls = h->d_clsA; g.plain = h->d_plainA; g.nplain = h->nplainA;
         scatter_to(h, g, h->d_tilesA, h->ntilesA, 1, h->stA, (size_t)ns0 * h->P * N, s);
         lpk::launch_scatter_extra(h->d_G, acc, ns0, h->Nt, h->Nr, N, h->P, h->d_xrow, h->d_xent, h->cubic, s);
     }

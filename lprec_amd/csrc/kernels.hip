@@ -2138,16 +2138,13 @@ __global__ void __launch_bounds__(kGatherThreads) k_scatter(Scatter g, const GTi
     const int nzg = (g.nz + g.zgroup - 1) / g.zgroup;
     const int lbk = xcd_block(blockIdx.x, gridDim.x);
     const int ng = gridDim.x / nzg;
-    const int zg = lbk % nzg, tile = (int)(((long long)(lbk / nzg) * g.tstride) % ng);
+    // (with colours: the groups that hold an uncoloured tile; k_scatter_col handles the coloured ones)
+    const int zg = lbk % nzg;
+    const int tile = g.perm ? g.plain[lbk / nzg] : (int)(((long long)(lbk / nzg) * g.tstride) % ng);
     const GTile* tb = tiles + (size_t)tile * g.group;
     const GTile t0 = tb[0];
     const int npts = t0.nr * t0.nc;
     const int z0 = zg * g.zgroup, z1 = min(z0 + g.zgroup, g.nz);
-    if (g.perm) {   // k_scatter_col handles the coloured tiles
-        bool any = false;
-        for (int gi = 0; gi < g.group; ++gi) any |= tb[gi].bw > 0 && tb[gi].cr == 0;
-        if (!any) return;
-    }
     // Loads are unconditional at clamped point indices (a guarded load
     // compiles to a branch and a wait of its own), all PPT in flight at once.
     const float inv_nc0 = 1.0f / (float)t0.nc;
@@ -2294,14 +2291,15 @@ void launch_zero(float* p, size_t n, hipStream_t s) {
 // class have disjoint tap footprints, so each box word takes at most one
 // plain read-modify-write per class -- no atomics, and the order of the
 // additions is fixed.  Same block order, boxes and flush as k_scatter.
+// A class has ~80 points and is bound by latency, not by work: a lane's point
+// index is loaded two classes ahead and its coordinate, value and scale one
+// class ahead, and the barrier between classes waits for LDS traffic only
+// (image -> LP transpose, N = 1024, 16 slices: 391 us, 690 with the loads
+// in the class and 256 threads).
 template <int KIND>
-__global__ void __launch_bounds__(kGatherThreads) k_scatter_col(Scatter g, const GTile* __restrict__ tiles) {
+__global__ void __launch_bounds__(kScatterThreads) k_scatter_col(Scatter g, const GTile* __restrict__ tiles) {
     extern __shared__ float box[];
-    // KZ slices share each pass over the colour classes: a point's tap
-    // geometry is computed once and added into KZ boxes (one per slice, LDS
-    // KZ * box_floats), so the block has half the class barriers per slice
-    constexpr int KZ = kScatterSlices;
-    const int nt = blockDim.x;
+    constexpr int nt = kScatterThreads;
     const int nzg = (g.nz + g.zgroup - 1) / g.zgroup;
     const int lbk = xcd_block(blockIdx.x, gridDim.x);
     const int ng = gridDim.x / nzg;
@@ -2309,95 +2307,104 @@ __global__ void __launch_bounds__(kGatherThreads) k_scatter_col(Scatter g, const
     const GTile* tb = tiles + (size_t)tile * g.group;
     const GTile t0 = tb[0];
     const int z0 = zg * g.zgroup, z1 = min(z0 + g.zgroup, g.nz);
-    const int bstride = g.box_floats;
-    for (int zb = z0; zb < z1; zb += KZ) {
-        const int zn = min(KZ, z1 - zb);
-        const float* V = g.val + (size_t)zb * g.v_z + (size_t)t0.span * g.v_span;
+    const int tid = threadIdx.x;
+    struct Point {
+        float2 c;
+        float v, sc;
+    };
+    for (int z = z0; z < z1; ++z) {
+        const float* V = g.val + (size_t)z * g.v_z + (size_t)t0.span * g.v_span + (size_t)t0.r0 * g.v_row + t0.c0;
         for (int gi = 0; gi < g.group; ++gi) {
             const GTile t = tb[gi];
             if (t.bw <= 0 || t.cr == 0) continue;   // uniform over the block
             const int bs = t.bs;
             const int nbox = bs * t.bh;
-            const float2* cb = g.coord + (size_t)t.span * g.c_span;
-            for (int q = 0; q < zn; ++q)
-                for (int i = threadIdx.x; i < nbox; i += nt) box[q * bstride + i] = 0.f;
-            __syncthreads();
+            const float2* cb = g.coord + (size_t)t.span * g.c_span + (size_t)(t.r0 + g.c_ro) * g.c_row + t.c0 + g.c_co;
+            const float* sb = g.scale ? g.scale + (size_t)t0.r0 * g.s_row + t0.c0 : nullptr;
             const int ncol = t.cr * t.cc;
-            for (int col = 0; col < ncol; ++col) {
-                const int pb = g.cls[t.cbase + col], pe = g.cls[t.cbase + col + 1];
-#pragma unroll 1
-                for (int i = pb + (int)threadIdx.x; i < pe; i += nt) {
-                    const int p = g.perm[t.pbase + i];
-                    const int r = p >> t.lnc, cidx = p & (t.nc - 1);
-                    const float2 c = cb[(size_t)(t.r0 + r + g.c_ro) * g.c_row + t.c0 + cidx + g.c_co];
-                    const size_t vo = (size_t)(t0.r0 + r) * g.v_row + t0.c0 + cidx;
-                    const float sc = g.scale ? g.scale[(size_t)(t0.r0 + r) * g.s_row + t0.c0 + cidx] : 1.f;
-                    float v[KZ];
+            const int* cls = g.cls + t.cbase;
+            const unsigned short* perm = g.perm + t.pbase;
+            const int npt = cls[ncol];
+            // (lanes past the end of the list, or of a class, load a valid
+            // point's data and drop it)
+            auto index = [&](int i) { return (int)perm[min(i, npt - 1)]; };
+            auto fetch = [&](int p) {
+                Point q;
+                const int r = p >> t.lnc, cidx = p & (t.nc - 1);
+                q.c = ld_at(cb, (unsigned)(r * g.c_row + cidx) * 8u);
+                q.v = ld_at(V, (unsigned)(r * g.v_row + cidx) * 4u);
+                q.sc = sb ? ld_at(sb, (unsigned)(r * g.s_row + cidx) * 4u) : 1.f;
+                return q;
+            };
+            auto deposit = [&](const Point& q) {
+                const float v = q.v * q.sc;
+                const float fx = floorf(q.c.x), fy = floorf(q.c.y);
+                const float ax = q.c.x - fx, ay = q.c.y - fy;
+                const int lx = min(max((int)fx - 1 - t.x0, 0), t.bw - 4);
+                const int ly = min(max((int)fy - 1 - t.y0, 0), t.bh - 4);
+                float* qb = box + ly * bs + lx;
+                if (g.cubic) {
+                    float wx[4], wy[4];
+                    bspline_w(ax, wx);
+                    bspline_w(ay, wy);
+                    float s[4][4];
 #pragma unroll
-                    for (int q = 0; q < KZ; ++q) v[q] = q < zn ? V[vo + (size_t)q * g.v_z] : 0.f;
-                    if (g.scale) {
+                    for (int b = 0; b < 4; ++b)
 #pragma unroll
-                        for (int q = 0; q < KZ; ++q) v[q] *= sc;
+                        for (int a = 0; a < 4; ++a) s[b][a] = qb[b * bs + a];
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        const float vb = wy[b] * v;
+#pragma unroll
+                        for (int a = 0; a < 4; ++a) qb[b * bs + a] = s[b][a] + wx[a] * vb;
                     }
-                    const float fx = floorf(c.x), fy = floorf(c.y);
-                    const float ax = c.x - fx, ay = c.y - fy;
-                    const int lx = min(max((int)fx - 1 - t.x0, 0), t.bw - 4);
-                    const int ly = min(max((int)fy - 1 - t.y0, 0), t.bh - 4);
-                    if (g.cubic) {
-                        float wx[4], wy[4];
-                        bspline_w(ax, wx);
-                        bspline_w(ay, wy);
-#pragma unroll
-                        for (int q = 0; q < KZ; ++q) {
-                            if (q >= zn) break;
-                            float* qb = box + q * bstride + ly * bs + lx;
-#pragma unroll
-                            for (int b = 0; b < 4; ++b) {
-                                const float vb = wy[b] * v[q];
-                                float* qr = qb + b * bs;
-                                const float s0 = qr[0], s1 = qr[1], s2 = qr[2], s3 = qr[3];
-                                qr[0] = s0 + wx[0] * vb;
-                                qr[1] = s1 + wx[1] * vb;
-                                qr[2] = s2 + wx[2] * vb;
-                                qr[3] = s3 + wx[3] * vb;
-                            }
-                        }
-                    } else {
-#pragma unroll
-                        for (int q = 0; q < KZ; ++q) {
-                            if (q >= zn) break;
-                            float* q1 = box + q * bstride + ly * bs + lx + bs + 1;
-                            float* q2 = q1 + bs;
-                            q1[0] += (1.f - ay) * (1.f - ax) * v[q];
-                            q1[1] += (1.f - ay) * ax * v[q];
-                            q2[0] += ay * (1.f - ax) * v[q];
-                            q2[1] += ay * ax * v[q];
-                        }
-                    }
+                } else {
+                    float* q1 = qb + bs + 1;
+                    float* q2 = q1 + bs;
+                    q1[0] += (1.f - ay) * (1.f - ax) * v;
+                    q1[1] += (1.f - ay) * ax * v;
+                    q2[0] += ay * (1.f - ax) * v;
+                    q2[1] += ay * ax * v;
                 }
-                __syncthreads();
+            };
+            // class bounds of the classes k, k + 1, k + 2 (scalar)
+            int b0 = 0, b1 = cls[1], b2 = cls[min(2, ncol)];
+            int pn = index(b0 + tid);
+            Point cur = fetch(pn);
+            pn = index(b1 + tid);   // class 1
+            for (int i = tid; i < nbox; i += nt) box[i] = 0.f;
+            lds_barrier();
+            for (int col = 0; col < ncol; ++col) {
+                const int b3 = cls[min(col + 3, ncol)];
+                const Point nxt = fetch(pn);      // class col + 1
+                pn = index(b2 + tid);             // class col + 2
+                if (b0 + tid < b1) deposit(cur);
+#pragma unroll 1
+                for (int i = b0 + tid + nt; i < b1; i += nt) deposit(fetch(index(i)));
+                lds_barrier();
+                cur = nxt;
+                b0 = b1;
+                b1 = b2;
+                b2 = b3;
             }
             const float inv = 1.0f / (float)t.bw;
             const int nb = t.bw * t.bh;
-            for (int q = 0; q < zn; ++q) {
-                const float* bq = box + q * bstride;
-                if (g.stage) {
-                    float* B = g.stage + (size_t)(zb + q) * g.stage_z + g.box_off[(size_t)tile * g.group + gi];
-                    for (int i = threadIdx.x; i < nb; i += nt) {
-                        const int yy = (int)(((float)i + 0.5f) * inv);
-                        B[i] = bq[yy * bs + (i - yy * t.bw)];
-                    }
-                } else {
-                    float* D = g.dst + (size_t)(zb + q) * g.dst_z + (size_t)t.span * g.dst_span;
-                    for (int i = threadIdx.x; i < nb; i += nt) {
-                        const int yy = (int)(((float)i + 0.5f) * inv);
-                        const int xx = i - yy * t.bw;
-                        const float v = bq[yy * bs + xx];
-                        if (v != 0.f) unsafeAtomicAdd(D + (size_t)wrapi(t.y0 + yy, g.H) * g.W + wrapi(t.x0 + xx, g.W), v);
-                    }
+            if (g.stage) {
+                float* B = g.stage + (size_t)z * g.stage_z + g.box_off[(size_t)tile * g.group + gi];
+                for (int i = tid; i < nb; i += nt) {
+                    const int yy = (int)(((float)i + 0.5f) * inv);
+                    B[i] = box[yy * bs + (i - yy * t.bw)];
+                }
+            } else {
+                float* D = g.dst + (size_t)z * g.dst_z + (size_t)t.span * g.dst_span;
+                for (int i = tid; i < nb; i += nt) {
+                    const int yy = (int)(((float)i + 0.5f) * inv);
+                    const int xx = i - yy * t.bw;
+                    const float v = box[yy * bs + xx];
+                    if (v != 0.f) unsafeAtomicAdd(D + (size_t)wrapi(t.y0 + yy, g.H) * g.W + wrapi(t.x0 + xx, g.W), v);
                 }
             }
-            __syncthreads();
+            lds_barrier();
         }
     }
 }
@@ -2416,13 +2423,14 @@ void launch_scatter(const Scatter& g0, const GTile* tiles, int ntiles, int kind,
     dim3 grid(ng * ((g.nz + g.zgroup - 1) / g.zgroup));
     size_t lds = (size_t)g.box_floats * sizeof(float);
     if (g.perm) {
-        const size_t ldsc = lds * kScatterSlices;
         switch (kind) {
-            case 0: hipLaunchKernelGGL(k_scatter_col<0>, grid, dim3(kGatherThreads), ldsc, s, g, tiles); break;
-            case 1: hipLaunchKernelGGL(k_scatter_col<1>, grid, dim3(kGatherThreads), ldsc, s, g, tiles); break;
-            case 2: hipLaunchKernelGGL(k_scatter_col<2>, grid, dim3(kGatherThreads), ldsc, s, g, tiles); break;
-            default: hipLaunchKernelGGL(k_scatter_col<3>, grid, dim3(kGatherThreads), ldsc, s, g, tiles); break;
+            case 0: hipLaunchKernelGGL(k_scatter_col<0>, grid, dim3(kScatterThreads), lds, s, g, tiles); break;
+            case 1: hipLaunchKernelGGL(k_scatter_col<1>, grid, dim3(kScatterThreads), lds, s, g, tiles); break;
+            case 2: hipLaunchKernelGGL(k_scatter_col<2>, grid, dim3(kScatterThreads), lds, s, g, tiles); break;
+            default: hipLaunchKernelGGL(k_scatter_col<3>, grid, dim3(kScatterThreads), lds, s, g, tiles); break;
         }
+        if (g.nplain <= 0) return;
+        grid.x = g.nplain * ((g.nz + g.zgroup - 1) / g.zgroup);
     }
     switch (kind) {
         case 0: hipLaunchKernelGGL(k_scatter<0>, grid, dim3(kGatherThreads), lds, s, g, tiles); break;
@@ -2435,6 +2443,7 @@ void launch_scatter(const Scatter& g0, const GTile* tiles, int ntiles, int kind,
 // Step A of the polar transpose: a block of 256 rows of one (span, angle);
 // the rows' detector runs are consecutive, so the coordinate and value loads
 // of neighbouring lanes are too.  u [nz][3][nA][Nrho].
+template <int ZC>
 __global__ void __launch_bounds__(256) k_polarT_rows(PolarT p) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     const int al = blockIdx.y, k = blockIdx.z;
@@ -2458,11 +2467,19 @@ __global__ void __launch_bounds__(256) k_polarT_rows(PolarT p) {
         const int b0 = xa[max(lo, 0)], b1 = xa[min(hi, p.Q)];
         if (b0 < b1) { x0[nq] = b0; x1[nq] = b1; qq[nq] = q; ++nq; }
     }
-    for (int z = 0; z < p.nz; ++z) {
-        const float* V = p.val + (size_t)z * p.v_z + (size_t)a * p.N0;
-        float acc = 0.f;
+    // a cell's weight is formed once per ZC slices, whose values are in flight
+    // together (one slice at a time: 193 us at N = 1024, 16 slices; 8: 81)
+    for (int z0 = 0; z0 < p.nz; z0 += ZC) {
+        const float* V = p.val + (size_t)z0 * p.v_z + (size_t)a * p.N0;
+        const int zn = min(ZC, p.nz - z0);
+        float acc[ZC];
+#pragma unroll
+        for (int q = 0; q < ZC; ++q) acc[q] = 0.f;
         for (int t = 0; t < nq; ++t)
             for (int x = x0[t]; x < x1[t]; ++x) {
+                float v[ZC];
+#pragma unroll
+                for (int q = 0; q < ZC; ++q) v[q] = V[(size_t)min(q, zn - 1) * p.v_z + x];
                 const float y = ca[x].y;
                 const float fy = floorf(y);
                 const int b = qq[t] - (int)fy + (p.cubic ? 1 : 0);
@@ -2475,18 +2492,27 @@ __global__ void __launch_bounds__(256) k_polarT_rows(PolarT p) {
                 } else {
                     w = b == 0 ? 1.f - ay : ay;
                 }
-                acc += w * V[x];
+#pragma unroll
+                for (int q = 0; q < ZC; ++q) acc[q] += w * v[q];
             }
-        U[z * u_z] = acc;
+#pragma unroll
+        for (int q = 0; q < ZC; ++q)
+            if (q < zn) U[(size_t)(z0 + q) * u_z] = acc[q];
     }
 }
 
-// Step B: a block owns 64 columns x 64 rows of one span; the u rows of the
-// angles whose taps reach those columns are staged through LDS 128 angles at
-// a time, and each lane sums its column for 16 rows.
+// Step B: a block owns 64 columns x 64 rows of one span and a few slices; the
+// u rows of the angles whose taps reach those columns are staged through LDS
+// 128 angles at a time, and each lane sums its column for 16 rows.  A column
+// has about 4 P0 / 1.5 N angles: the weights of up to 8 are formed once per
+// block (formed per slice they took most of the kernel: 184 us at N = 1024,
+// 16 slices, 86 now).
+constexpr int kPolarTSlices = 4;
 __global__ void __launch_bounds__(256) k_polarT_cols(PolarT p) {
     __shared__ float us[128][65];
-    const int k = blockIdx.z, r0 = blockIdx.y * 64, jj0 = blockIdx.x * 64;
+    const int nzg = (p.nz + kPolarTSlices - 1) / kPolarTSlices;
+    const int k = blockIdx.z / nzg, z0 = (blockIdx.z - k * nzg) * kPolarTSlices, z1 = min(z0 + kPolarTSlices, p.nz);
+    const int r0 = blockIdx.y * 64, jj0 = blockIdx.x * 64;
     const int lc = threadIdx.x & 63, lr = threadIdx.x >> 6;
     const int jj = jj0 + lc, j = p.jlo + jj;
     const int* A = p.aj + (size_t)k * (p.jn + 5);
@@ -2498,7 +2524,25 @@ __global__ void __launch_bounds__(256) k_polarT_cols(PolarT p) {
     const int a0 = p.abeg[k];
     const size_t u_z = (size_t)3 * p.nA * p.Nr;
     const size_t g_z = (size_t)p.Nr * p.Nt;
-    for (int z = 0; z < p.nz; ++z) {
+    auto weight = [&](int al) {
+        const float x = p.cxa[a0 + al];
+        const float fx = floorf(x);
+        const int c = j - (int)fx + (p.cubic ? 1 : 0);
+        const float ax = x - fx;
+        if (p.cubic) {
+            float wx[4];
+            bspline_w(ax, wx);
+            return c == 0 ? wx[0] : c == 1 ? wx[1] : c == 2 ? wx[2] : wx[3];
+        }
+        return c == 0 ? 1.f - ax : ax;
+    };
+    constexpr int NW = 8;
+    float wh[NW];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) wh[i] = lo + i < hi ? weight(lo + i) : 0.f;
+    // one staging covers the block's angles, and every lane has few
+    const bool held = bhi - blo <= 128 && !__syncthreads_or(hi - lo > NW);
+    for (int z = z0; z < z1; ++z) {
         float acc[16];
 #pragma unroll
         for (int m = 0; m < 16; ++m) acc[m] = 0.f;
@@ -2506,27 +2550,34 @@ __global__ void __launch_bounds__(256) k_polarT_cols(PolarT p) {
         for (int c0 = blo; c0 < bhi; c0 += 128) {
             const int cn = min(128, bhi - c0);
             __syncthreads();
-            for (int i = threadIdx.x; i < cn * 64; i += blockDim.x) {
-                const int ai = i >> 6, ri = i & 63;
-                const int rr = r0 + ri;
-                us[ai][ri] = rr < p.Nr ? U[(size_t)(c0 + ai) * p.Nr + rr] : 0.f;
-            }
-            __syncthreads();
-            for (int al = max(lo, c0); al < min(hi, c0 + cn); ++al) {
-                const float x = p.cxa[a0 + al];
-                const float fx = floorf(x);
-                const int c = j - (int)fx + (p.cubic ? 1 : 0);
-                const float ax = x - fx;
-                float w;
-                if (p.cubic) {
-                    float wx[4];
-                    bspline_w(ax, wx);
-                    w = c == 0 ? wx[0] : c == 1 ? wx[1] : c == 2 ? wx[2] : wx[3];
-                } else {
-                    w = c == 0 ? 1.f - ax : ax;
+            for (int i0 = threadIdx.x; i0 < cn * 64; i0 += 8 * 256) {
+                float v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int i = min(i0 + u * 256, cn * 64 - 1);
+                    v[u] = U[(size_t)(c0 + (i >> 6)) * p.Nr + min(r0 + (i & 63), p.Nr - 1)];
                 }
 #pragma unroll
-                for (int m = 0; m < 16; ++m) acc[m] += w * us[al - c0][lr + 4 * m];
+                for (int u = 0; u < 8; ++u) {
+                    const int i = min(i0 + u * 256, cn * 64 - 1);
+                    us[i >> 6][i & 63] = v[u];   // (rows past Nr are not stored below)
+                }
+            }
+            __syncthreads();
+            if (held) {
+#pragma unroll
+                for (int i = 0; i < NW; ++i) {
+                    if (lo + i < hi) {
+#pragma unroll
+                        for (int m = 0; m < 16; ++m) acc[m] += wh[i] * us[lo + i - c0][lr + 4 * m];
+                    }
+                }
+            } else {
+                for (int al = max(lo, c0); al < min(hi, c0 + cn); ++al) {
+                    const float w = weight(al);
+#pragma unroll
+                    for (int m = 0; m < 16; ++m) acc[m] += w * us[al - c0][lr + 4 * m];
+                }
             }
         }
         if (jj < p.jn) {
@@ -2541,17 +2592,25 @@ __global__ void __launch_bounds__(256) k_polarT_cols(PolarT p) {
 }
 
 void launch_polar_transpose(const PolarT& p, hipStream_t s) {
-    hipLaunchKernelGGL(k_polarT_rows, dim3((p.Nr + 255) / 256, p.nA, 3), dim3(256), 0, s, p);
-    hipLaunchKernelGGL(k_polarT_cols, dim3((p.jn + 63) / 64, (p.Nr + 63) / 64, 3), dim3(256), 0, s, p);
+    const dim3 ga((p.Nr + 255) / 256, p.nA, 3);
+    if (p.nz >= 5) hipLaunchKernelGGL(k_polarT_rows<8>, ga, dim3(256), 0, s, p);
+    else if (p.nz >= 2) hipLaunchKernelGGL(k_polarT_rows<4>, ga, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL(k_polarT_rows<1>, ga, dim3(256), 0, s, p);
+    hipLaunchKernelGGL(k_polarT_cols, dim3((p.jn + 63) / 64, (p.Nr + 63) / 64, 3 * ((p.nz + kPolarTSlices - 1) / kPolarTSlices)),
+                       dim3(256), 0, s, p);
 }
 
-// One block per destination tile of 32 x 32 points (4 per thread); the
-// tile's box list is walked once per 8 slices, its rectangles and offsets
-// staged in LDS 128 at a time (one burst of list reads instead of a
-// dependent pair of global loads per box), and two boxes' value loads are in
-// flight together.  Every point adds its boxes in list order.
+// One block per destination tile of 32 x 32 points (4 per thread) and ZC
+// slices; the tile's box list is walked once, its rectangles and offsets
+// staged in LDS 128 at a time (one burst of list reads instead of a dependent
+// pair of global loads per box).  The 32 values of a box are loaded
+// unconditionally at offsets clamped into it and masked afterwards, so they
+// travel together (guarded loads waited one by one: 385 us at N = 1024, 16
+// slices, 128 now); boxes that miss a wave's points are skipped.  Every point adds its
+// boxes in list order.
+template <int ZC>
 __global__ void __launch_bounds__(256) k_box_sum(BoxSum b) {
-    constexpr int ZC = 8, LB = 128;
+    constexpr int LB = 128;
     __shared__ int4 srect[LB];
     __shared__ int soff[LB];
     const int t = blockIdx.x;
@@ -2561,60 +2620,72 @@ __global__ void __launch_bounds__(256) k_box_sum(BoxSum b) {
     const int X = tx * 32 + (threadIdx.x & 31);
     const int Y0 = ty * 32 + (threadIdx.x >> 5);   // rows Y0 + 8 e, e < 4
     const int beg = b.tile_beg[t], end = b.tile_beg[t + 1];
-    for (int z0 = 0; z0 < b.nz; z0 += ZC) {
-        const int zn = min(ZC, b.nz - z0);
-        float acc[ZC][4];
+    const int z0 = blockIdx.y * ZC, zn = min(ZC, b.nz - z0);
+    float acc[ZC][4];
 #pragma unroll
-        for (int q = 0; q < ZC; ++q)
+    for (int q = 0; q < ZC; ++q)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[q][e] = 0.f;
-        const float* St = b.stage + (size_t)z0 * b.stage_z;
-        for (int c0 = beg; c0 < end; c0 += LB) {
-            const int nb = min(LB, end - c0);
-            __syncthreads();   // the previous round's entries are read
-            if ((int)threadIdx.x < nb) {
-                const int id = b.tile_box[c0 + threadIdx.x];
-                srect[threadIdx.x] = b.box_rect[id];
-                soff[threadIdx.x] = b.box_off[id];
-            }
-            __syncthreads();
-#pragma unroll 2
-            for (int i = 0; i < nb; ++i) {
-                const int4 r = srect[i];
-                const float* B = St + soff[i];
-                // box origins lie within one period of the plane: one wrap at most
-                int dx = X - r.x;
-                dx += dx < 0 ? b.W : (dx >= b.W ? -b.W : 0);
-                if (dx >= r.z) continue;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    int dy = Y0 + 8 * e - r.y;
-                    dy += dy < 0 ? b.H : (dy >= b.H ? -b.H : 0);
-                    if (dy < r.w) {
-                        const float* Bq = B + dy * r.z + dx;
-#pragma unroll
-                        for (int q = 0; q < ZC; ++q)
-                            if (q < zn) acc[q][e] += Bq[(size_t)q * b.stage_z];
-                    }
-                }
-            }
+        for (int e = 0; e < 4; ++e) acc[q][e] = 0.f;
+    const float* St = b.stage + (size_t)z0 * b.stage_z;
+    for (int c0 = beg; c0 < end; c0 += LB) {
+        const int nb = min(LB, end - c0);
+        __syncthreads();   // the previous round's entries are read
+        if ((int)threadIdx.x < nb) {
+            const int id = b.tile_box[c0 + threadIdx.x];
+            srect[threadIdx.x] = b.box_rect[id];
+            soff[threadIdx.x] = b.box_off[id];
         }
-#pragma unroll
-        for (int q = 0; q < ZC; ++q) {
-            if (q >= zn) break;
-            float* D = b.dst + (size_t)(z0 + q) * b.dst_z + (size_t)plane * b.dst_plane;
+        __syncthreads();
+        for (int i = 0; i < nb; ++i) {
+            const int4 r = srect[i];
+            const float* B = St + soff[i];
+            // box origins lie within one period of the plane: one wrap at most
+            int dx = X - r.x;
+            dx += dx < 0 ? b.W : (dx >= b.W ? -b.W : 0);
+            bool ok[4], any = false;
+            unsigned off[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int Y = Y0 + 8 * e;
-                if (X < b.W && Y < b.H) D[(size_t)Y * b.W + X] = acc[q][e];
+                int dy = Y0 + 8 * e - r.y;
+                dy += dy < 0 ? b.H : (dy >= b.H ? -b.H : 0);
+                ok[e] = dx < r.z && dy < r.w;
+                any |= ok[e];
+                off[e] = ok[e] ? (unsigned)(dy * r.z + dx) * 4u : 0u;
             }
+            if (!__any(any)) continue;
+            float v[ZC][4];
+#pragma unroll
+            for (int q = 0; q < ZC; ++q) {
+                const float* Bq = B + (size_t)min(q, zn - 1) * b.stage_z;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[q][e] = ld_at(Bq, off[e]);
+            }
+#pragma unroll
+            for (int q = 0; q < ZC; ++q)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[q][e] += ok[e] ? v[q][e] : 0.f;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < ZC; ++q) {
+        if (q >= zn) break;
+        float* D = b.dst + (size_t)(z0 + q) * b.dst_z + (size_t)plane * b.dst_plane;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int Y = Y0 + 8 * e;
+            if (X < b.W && Y < b.H) D[(size_t)Y * b.W + X] = acc[q][e];
         }
     }
 }
 
 void launch_box_sum(const BoxSum& b, hipStream_t s) {
     const int nt = b.nplanes * b.tiles_x * b.tiles_y;
-    if (nt > 0) hipLaunchKernelGGL(k_box_sum, dim3(nt), dim3(256), 0, s, b);
+    if (nt <= 0) return;
+    // (fewer slices per block on small planes gave nothing: N = 256, 4 slices
+    // and N = 512, 8 slices the same from 1 to 8)
+    if (b.nz >= 5) hipLaunchKernelGGL(k_box_sum<8>, dim3(nt, (b.nz + 7) / 8), dim3(256), 0, s, b);
+    else if (b.nz >= 2) hipLaunchKernelGGL(k_box_sum<4>, dim3(nt), dim3(256), 0, s, b);
+    else hipLaunchKernelGGL(k_box_sum<1>, dim3(nt), dim3(256), 0, s, b);
 }
 
 void launch_scatter_extra(const float* F, float* dst, int nz, int Ntheta, int Nrho, int W, int H, const int* xrow,

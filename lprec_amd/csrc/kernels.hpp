@@ -199,11 +199,11 @@ struct Gather {
     int nz, zgroup, group, cubic, box_floats;
 };
 constexpr int kGatherThreads = 256;
+// threads of the coloured scatter: a colour class holds ~80 points of a tile,
+// and more blocks fit a compute unit (fwd_T / adj_T, N = 1024, 16 slices:
+// 64 threads 1355 / 2188 us, 128 1254 / 1944, 256 1302 / 2034)
+constexpr int kScatterThreads = 128;
 constexpr int kGatherPPT = 8;   // points per thread: tiles hold <= 2048 points
-// slices per colour pass of the coloured scatter (k_scatter_col); 2 measured
-// no faster (0.692 against 0.699 ms per call, N0 = 1024, 16 slices) for
-// twice the LDS
-constexpr int kScatterSlices = 1;
 #ifndef LP_GATHER_PIPE
 #define LP_GATHER_PIPE 2
 #endif
@@ -242,6 +242,8 @@ struct Scatter {
     const int* box_off;
     const unsigned short* perm;   // colour-sorted points of the tiles (GTile.pbase)
     const int* cls;               // colour class bounds (GTile.cbase)
+    const int* plain;             // with perm: the nplain tile groups that hold an uncoloured tile
+    int nplain;
 };
 // Destination of staged scatter boxes: dst tiles of 32 x 32 points, each the
 // sum, in increasing box order, of the staged boxes that cover it (periodic
