@@ -1591,71 +1591,111 @@ __device__ __forceinline__ void dft32(float2* v, int dir) {
     }
 }
 
-// Inverse row pass at h = 1024 (Ntheta = 2048) with 32 lanes per row: a lane
-// holds 32 elements, so the length-1024 FFT is one register DFT32 over
-// elements 32 apart, the twiddles W1024^(l m), one LDS exchange within the
-// row and a second register DFT32 (1024 = 32 x 32).  16 rows per 512-lane
-// block (the transposed half-spectra are read in 128-byte segments); at 512
-// lanes a lane has 256 VGPRs, which hold the next slice's 32 loads while the
-// current slice is transformed and stored.  S is read and G written with the
-// non-temporal hint.  (The same scheme for the forward row pass measured
-// slower than k_rows16_fwd, with or without the prefetch.)
-// LDS: 16 rows at stride 1090 slots (the layout of k_rows16_*), then the
-// twiddles W1024^(l m) at [m * 32 + l] (a fixed m is read conflict-free by
-// the 32 lanes l) and twN[0, 512].
-constexpr int kRows32RS = 1024 + 1024 / 16 + 2;
-constexpr size_t kRows32Lds = (size_t)(16 * kRows32RS + 1024 + 513) * sizeof(float2);
+// Inverse row pass at h = 1024 and 2048 with half a wave or a wave per row: a
+// lane holds 32 elements x[l + LPR q], so the transform is one register DFT32
+// over q, the twiddles, one LDS exchange within the row and a second register
+// transform -- no block barrier but the two around the transposed copy.  512
+// lanes, 16 or 8 rows per block (the transposed half-spectra are read in 128-
+// or 64-byte segments); a lane's 256 VGPRs hold the next slice's 32 loads
+// while the current slice is transformed and stored.  S is read and G written
+// with the non-temporal hint.  At h = 2048, N = 4096 (600 MB): 1 slice 246 us,
+// 4 slices 755, against 323 and 1034 for the radix-16 kernel, whose 1024 lanes
+// meet at a barrier in every stage.  (The same scheme for the forward row pass
+// measured no faster than k_rows16_fwd: 227 against 214 us at h = 2048, 1.23
+// against 1.03 ms at h = 1024, 32 slices.)
+// LDS: the rows (stride RS, the layout of k_rows16_*), the twiddles
+// W_H^(l m), m > 0, at [(m - 1) * LPR + l] and twN[0, H/2]: at h = 2048 all
+// 160 KB.
+template <int H>
+struct RowsWave {
+    static constexpr int LPR = H / 32, R = 512 / LPR, RS = H + H / 16 + 32 / R;
+    static constexpr size_t lds = (size_t)(R * RS + H - LPR + H / 2 + 1) * sizeof(float2);
+    static_assert(lds <= 163840, "LDS of a compute unit");
+};
 
-__device__ __forceinline__ void rows32_tables(float2* tw2, float2* twn, const RowPass& rp) {
-    for (int i = threadIdx.x; i < 1024; i += 512) tw2[i] = rp.twh[(i & 31) * (i >> 5)];
-    for (int i = threadIdx.x; i <= 512; i += 512) twn[i] = rp.twN[i];
-}
-
-// Length-1024 FFT of the row owned by lanes li = 0..31 of one wave half,
-// v[q] = x[li + 32 q] on entry, v[k] = X[li + 32 k] on exit.  The exchange
-// goes through the row's slots m * 33 + l (m, l < 32; the odd stride keeps
-// both the writes, fixed m, and the reads, fixed l, free of bank
-// conflicts), which must be free on entry and are free again on exit.
-__device__ __forceinline__ void rows32_fft(float2* v, float2* row, const float2* tw2, int li, int dir) {
+// FFT of the row owned by lanes li = 0 .. LPR - 1, v[q] = x[li + LPR q] on
+// entry, v[k] = X[li + LPR k] on exit.  The exchange goes through the row's
+// slots m * (LPR + 1) + l (the odd stride keeps the writes, fixed m, and the
+// reads, fixed l, free of bank conflicts), which must be free on entry and are
+// free again on exit.  At 2048 a second transform has 64 points and two lanes,
+// which take its even and its odd outputs: both read all its inputs.
+template <int H>
+__device__ __forceinline__ void rows_wave_fft(float2* v, float2* row, const float2* tw2, int li, int dir) {
+    constexpr int LPR = RowsWave<H>::LPR, XS = LPR + 1;
     dft32(v, dir);
 #pragma unroll
     for (int m = 1; m < 32; ++m) {
-        const float2 w = tw2[m * 32 + li];
+        const float2 w = tw2[(m - 1) * LPR + li];
         v[m] = cmul(v[m], dir < 0 ? w : cconj(w));
     }
 #pragma unroll
-    for (int m = 0; m < 32; ++m) row[m * 33 + li] = v[m];
+    for (int m = 0; m < 32; ++m) row[m * XS + li] = v[m];
     wave_sync();
+    if constexpr (H == 1024) {
 #pragma unroll
-    for (int l = 0; l < 32; ++l) v[l] = row[li * 33 + l];
+        for (int l = 0; l < 32; ++l) v[l] = row[li * XS + l];
+    } else {
+        // cos and sin of pi l / 32
+        constexpr float C[32] = {1.0f, 0.99518472667219688624f, 0.98078528040323044913f, 0.95694033573220886494f,
+                                 0.92387953251128675613f, 0.88192126434835502971f, 0.83146961230254523708f,
+                                 0.77301045336273696081f, 0.70710678118654752440f, 0.63439328416364549822f,
+                                 0.55557023301960222474f, 0.47139673682599764856f, 0.38268343236508977173f,
+                                 0.29028467725446236764f, 0.19509032201612826785f, 0.09801714032956060199f, 0.0f,
+                                 -0.09801714032956060199f, -0.19509032201612826785f, -0.29028467725446236764f,
+                                 -0.38268343236508977173f, -0.47139673682599764856f, -0.55557023301960222474f,
+                                 -0.63439328416364549822f, -0.70710678118654752440f, -0.77301045336273696081f,
+                                 -0.83146961230254523708f, -0.88192126434835502971f, -0.92387953251128675613f,
+                                 -0.95694033573220886494f, -0.98078528040323044913f, -0.99518472667219688624f};
+        const float2* in = row + (li & 31) * XS;
+        const bool odd = li >= 32;
+        const float sg = odd ? -1.f : 1.f, d = (float)dir;
+#pragma unroll
+        for (int l = 0; l < 32; ++l) {
+            const float2 x = in[l], y = in[l + 32];
+            v[l] = make_float2(x.x + sg * y.x, x.y + sg * y.y);
+            if (l % 8 == 7) __builtin_amdgcn_sched_barrier(0);   // (all 64 reads ahead would not fit the registers)
+        }
+        if (odd) {
+            // (sin pi l / 32 = cos pi |l - 16| / 32)
+#pragma unroll
+            for (int l = 1; l < 32; ++l) v[l] = cmul(v[l], make_float2(C[l], d * C[l < 16 ? 16 - l : l - 16]));
+        }
+    }
     dft32(v, dir);
     wave_sync();   // the exchange slots are read before the caller reuses them
 }
 
-__global__ void __launch_bounds__(512) k_rows32_inv(RowPass rp, float* __restrict__ G,
-                                                    const int2* __restrict__ wrange) {
+template <int H>
+__global__ void __launch_bounds__(512) k_rows32_inv(RowPass rp, float* __restrict__ G, const int2* __restrict__ wrange) {
     extern __shared__ float2 smc[];
-    constexpr int H = 1024, T = 32, R = 16, RS = kRows32RS;
+    using C = RowsWave<H>;
+    constexpr int R = C::R, RS = C::RS, LPR = C::LPR;
     const int Nt = rp.Ntheta, Nr = rp.Nrho;
-    const int r = threadIdx.x >> 5, li = threadIdx.x & 31;
+    const int r = threadIdx.x / LPR, li = threadIdx.x & (LPR - 1);
     const int nrb = Nr / R, nzg = (rp.nz + rp.zgroup - 1) / rp.zgroup;
     const int lb = xcd_block(blockIdx.x, gridDim.x);
     const int row0 = (lb % nrb) * R, span = lb / (nrb * nzg);
     const int z0 = ((lb / nrb) % nzg) * rp.zgroup;
     const int z1 = min(z0 + rp.zgroup, rp.nz);
+    if (rp.out_rows) {
+        // no row of the block is read by the output gather (every wave looks at
+        // all of them: __syncthreads_or takes LDS, and none is left)
+        const int2 w = wrange ? wrange[(size_t)span * Nr + row0 + (threadIdx.x & (R - 1))] : make_int2(0, Nt);
+        if (!__any((max(w.x, 0) >> 1) < min((w.y + 1) >> 1, H))) return;
+    }
     const int2 wr = wrange ? wrange[(size_t)span * Nr + row0 + r] : make_int2(0, Nt);
     const int e0 = max(wr.x, 0) >> 1, e1 = min((wr.y + 1) >> 1, H);
-    if (rp.out_rows && !__syncthreads_or(e0 < e1)) return;
     float2* row = smc + r * RS;
     float2* tw2 = smc + R * RS;
-    float2* twn = tw2 + 1024;
-    rows32_tables(tw2, twn, rp);
-    // transposed load: thread (rr, f0) = (tid mod 16, tid / 16) loads
-    // frequencies f0 + 32 i of row rr
-    const int rr = threadIdx.x & (R - 1), f0 = threadIdx.x >> 4;
+    float2* twn = tw2 + H - LPR;
+    for (int i = threadIdx.x; i < H - LPR; i += 512) tw2[i] = rp.twh[(i & (LPR - 1)) * (i / LPR + 1)];
+    for (int i = threadIdx.x; i <= H / 2; i += 512) twn[i] = rp.twN[i];
+    // transposed load: thread (rr, f0) = (tid mod R, tid / R) loads
+    // frequencies f0 + LPR i of row rr
+    const int rr = threadIdx.x & (R - 1), f0 = threadIdx.x / R;
     const unsigned lane = (unsigned)(f0 * Nr + rr) * 8u;
     float2* dst = smc + rr * RS + lidx(f0);
-    const unsigned step = 32u * (unsigned)Nr * 8u;   // bytes between frequencies f0 + 32 i and f0 + 32 (i + 1)
+    const unsigned step = (unsigned)LPR * (unsigned)Nr * 8u;   // bytes between frequencies f0 + LPR i and the next
     auto load = [&](int z, float2* w) {
         const float2* in = rp.S + ((size_t)span * rp.nz + z) * H * (size_t)Nr + row0;
         unsigned off = lane;
@@ -1667,25 +1707,25 @@ __global__ void __launch_bounds__(512) k_rows32_inv(RowPass rp, float* __restric
     load(z0, nx);
     for (int z = z0; z < z1; ++z) {
 #pragma unroll
-        for (int i = 0; i < 32; ++i) dst[34 * i] = nx[i];
+        for (int i = 0; i < 32; ++i) dst[(LPR + LPR / 16) * i] = nx[i];
         lds_barrier();   // every row was written by the whole block (and the tables, first time)
         // the lane index, opaque per slice: the LDS addresses derived from it
         // are recomputed here instead of being held across the loop next to
         // the prefetched loads
         int l = li;
         asm volatile("" : "+v"(l));
-        c2r_pre_row<H, T>(row, twn, l);
+        c2r_pre_row<H, LPR>(row, twn, l);
         wave_sync();
 #pragma unroll
-        for (int q = 0; q < 32; ++q) v[q] = row[lidx(l + 32 * q)];
+        for (int q = 0; q < 32; ++q) v[q] = row[lidx(l + LPR * q)];
         wave_sync();   // the exchange slots overlap the row
         if (z + 1 < z1) load(z + 1, nx);   // in flight while this slice is transformed and stored
-        rows32_fft(v, row, tw2, l, +1);
-        // v[k] = x[li + 32 k]: only the columns the output gather reads
+        rows_wave_fft<H>(v, row, tw2, l, +1);
+        // v[k] = x[li + LPR k]: only the columns the output gather reads
         float2* out = reinterpret_cast<float2*>(G + ((((size_t)span * rp.nz + z) * Nr + row0 + r) * (size_t)Nt));
 #pragma unroll
         for (int k = 0; k < 32; ++k) {
-            const int e = l + 32 * k;
+            const int e = l + LPR * k;
             if (e >= e0 && e < e1) st_at_nt(out, (unsigned)e * 8u, v[k]);
         }
         lds_barrier();   // the next slice's staging overwrites every row
@@ -1928,8 +1968,10 @@ static int rows16_mid(const RowPass& rp) {
     if ((long long)rp.R * (h / 16) > 1024) return 0;
     return h / 256;
 }
-// the 32-lane inverse row kernel: FFT kernel family 2, h = 1024, 16 rows per block
-static bool rows32_applies(const RowPass& rp) { return rp.fft16 == 2 && rp.h == 1024 && rp.R == 16; }
+// the inverse row kernel with 32 elements per lane: FFT kernel family 2, h = 1024 with 16 rows per block or h = 2048 with 8
+static bool rows32_applies(const RowPass& rp) {
+    return rp.fft16 == 2 && ((rp.h == 1024 && rp.R == RowsWave<1024>::R) || (rp.h == 2048 && rp.R == RowsWave<2048>::R));
+}
 static size_t rows16_lds(const RowPass& rp) {
     // the rows, then (h <= 2048) the staged twiddles twh[0, h/2) and twN[0, h/2]
     const size_t tws = rp.h <= 2048 ? (size_t)(rp.h + 1) * sizeof(float2) : 0;
@@ -1950,9 +1992,9 @@ static size_t rows16_lds(const RowPass& rp) {
 
 // Slices per block, reduced for small batches so that a launch still has
 // enough blocks to fill the chip several times over.
-static RowPass fit_zgroup(const RowPass& in, long long blocks_per_slice) {
+static RowPass fit_zgroup(const RowPass& in, long long blocks_per_slice, int blocks = 2048) {
     RowPass rp = in;
-    while (rp.zgroup > 1 && blocks_per_slice * ((rp.nz + rp.zgroup - 1) / rp.zgroup) < 2048) rp.zgroup /= 2;
+    while (rp.zgroup > 1 && blocks_per_slice * ((rp.nz + rp.zgroup - 1) / rp.zgroup) < blocks) rp.zgroup /= 2;
     return rp;
 }
 
@@ -2011,8 +2053,16 @@ void launch_rows_inv(const RowPass& rp0, float* G, const int2* wrange, hipStream
     if (int mid = rows16_mid(rp)) {
         dim3 grid((rp.Nrho / rp.R) * 3 * ((rp.nz + rp.zgroup - 1) / rp.zgroup));
         if (rows32_applies(rp)) {
-            allow_lds(k_rows32_inv, kRows32Lds);
-            hipLaunchKernelGGL(k_rows32_inv, grid, dim3(512), kRows32Lds, s, rp, G, wrange);
+            // (one block per compute unit: 3 rounds of blocks, and slices to load ahead)
+            const RowPass rq = fit_zgroup(rp0, 3LL * (rp0.Nrho / rp0.R), 768);
+            const dim3 g((rq.Nrho / rq.R) * 3 * ((rq.nz + rq.zgroup - 1) / rq.zgroup));
+            if (rq.h == 1024) {
+                allow_lds(k_rows32_inv<1024>, RowsWave<1024>::lds);
+                hipLaunchKernelGGL(k_rows32_inv<1024>, g, dim3(512), RowsWave<1024>::lds, s, rq, G, wrange);
+            } else {
+                allow_lds(k_rows32_inv<2048>, RowsWave<2048>::lds);
+                hipLaunchKernelGGL(k_rows32_inv<2048>, g, dim3(512), RowsWave<2048>::lds, s, rq, G, wrange);
+            }
             return;
         }
         dim3 block(rp.R * (rp.h / 16));
