@@ -1033,7 +1033,7 @@ void rtc_build(lp_handle* h) {
         h->rtc_fn[0] = h->rtc_fn[1] = h->rtc_fn[2] = h->rtc_fn[3] = nullptr;
         h->rtc_pair_tried = false;
     }
-    const bool rows = !h->rtc_tried && !pow2_in(h->h, 256, 4096), cols = !h->rtc_tried && !pow2_in(h->Nr, 256, 4096);
+    const bool rows = !h->rtc_tried && !pow2_in(h->h, 256, 4096), cols = !h->rtc_tried && !pow2_in(h->Nr, 256, 8192);
     // the filtered pair pass has no register kernel at any length; when the
     // filter comes after the first build (lp_init_adj after lp_init_fwd), it
     // is a module of its own

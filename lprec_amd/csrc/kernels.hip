@@ -1260,6 +1260,164 @@ __global__ void __launch_bounds__(ColShape<MID>::NT, 2) k_cols_stream(RowPass rp
     }
 }
 
+// W32^q = (cos, sin) of pi q / 16 applied to v[q], q < 16
+__device__ __forceinline__ void turn32(float2* v, int dir) {
+    constexpr float C[16] = {1.0f, 0.98078528040323044913f, 0.92387953251128675613f, 0.83146961230254523708f,
+                             0.70710678118654752440f, 0.55557023301960222474f, 0.38268343236508977173f,
+                             0.19509032201612826785f, 0.0f, -0.19509032201612826785f, -0.38268343236508977173f,
+                             -0.55557023301960222474f, -0.70710678118654752440f, -0.83146961230254523708f,
+                             -0.92387953251128675613f, -0.98078528040323044913f};
+    const float d = (float)dir;
+#pragma unroll
+    for (int q = 1; q < 16; ++q)   // (sin pi q / 16 = cos pi |q - 8| / 16)
+        v[q] = q == 8 ? rot90(v[q], dir) : cmul(v[q], make_float2(C[q], d * C[q < 8 ? 8 - q : q - 8]));
+}
+
+// The streaming column pass at M = 8192 = 32 x 16 x 16, 512 lanes with 16
+// elements each; block order, stream and constants as in k_cols_stream.  Two
+// lanes share a radix-32 butterfly (its even and its odd outputs, both read
+// all inputs); it comes first, where it has no twiddles, and the inverse runs
+// the transposed stages backwards (twiddles after the butterfly), so that it
+// comes last there.  The two radix-16 stages keep one butterfly per lane.
+// One block per compute unit (136 KB of LDS).  N = 4096, 1 and 4 slices: 263
+// and 846 us, against 308 and 1076 for the compiled pass (16 x 16 x 16 x 2, two
+// blocks without a stream); 131 at the copy rate.
+__global__ void __launch_bounds__(512, 2) k_cols_stream32(RowPass rp, int items, const float2* __restrict__ twM,
+                                                          const float2* __restrict__ fzT) {
+    constexpr int M = 8192, T = 512;
+    __shared__ float2 buf[lds_slots(M)];
+    __shared__ __align__(16) float2 pre[M];
+    const int h = rp.h, tid = threadIdx.x;
+    const int ng = (3 * rp.nz + items - 1) / items;
+    const int lb = xcd_block(blockIdx.x, gridDim.x);
+    const int f = lb / ng;
+    const int i0 = (lb % ng) * items, i1 = min(i0 + items, 3 * rp.nz);
+    const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), ln = threadIdx.x & 63;
+    auto column = [&](int it) { return rp.S + ((size_t)it * h + f) * (size_t)M; };
+    // 128-row chunks outside the rows that carry data are zeros
+    auto prefetch = [&](int it, int span) {
+        const int2 ir = rp.in_rows ? rp.in_rows[span] : make_int2(0, M);
+        const int c_lo = ir.x >> 7, c_hi = (ir.y + 127) >> 7;
+#pragma unroll
+        for (int c0 = 0; c0 < M / 128; c0 += T / 64) {
+            const int ch = c0 + wv;
+            float2* dst = pre + ch * 128;
+            if (ch >= c_lo && ch < c_hi) load_lds16<true>(column(it) + ch * 128 + ln * 2, dst);
+            else *reinterpret_cast<float4*>(dst + ln * 2) = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    int span = __builtin_amdgcn_readfirstlane(i0 / rp.nz), left = (span + 1) * rp.nz - i0;   // columns left in the span
+    prefetch(i0, span);
+    // radix-32 butterfly of a lane and its half of the outputs; the sixteen
+    // lanes of the other half are the neighbours (broadcast reads, writes on
+    // distinct banks)
+    auto butterfly = [](int li) { return (li >> 5) * 16 + (li & 15); };
+    auto half = [](int li) { return (li >> 4) & 1; };
+    float2 wm[4], wl[4], kz[16];
+#pragma unroll
+    for (int l = 0; l < 4; ++l) {
+        wm[l] = twM[((tid & 31) * 16) << l];
+        wl[l] = twM[tid << l];
+    }
+    const float2* fz = fzT + (size_t)f * M;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) kz[q] = fzval(fz, tid + q * T, rp.conj);
+    unsigned smask[3];   // stored rows among lo + q M / 16
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        smask[k] = rp.out_bits ? rp.out_bits[k * T + butterfly(tid) + 256 * half(tid)] : 0xffffu;
+    for (int it = i0; it < i1; ++it) {
+        float2 v[16];
+        // the lane index, opaque per column: addresses are formed where they
+        // are used, not held across the columns (a spill's reloads would join
+        // the vector-memory counter of the stream)
+        int li = tid;
+        asm volatile("" : "+v"(li));
+#pragma unroll
+        for (int l = 0; l < 4; ++l)   // (nor the products of one stage's twiddles)
+            asm volatile("" : "+v"(wl[l].x), "+v"(wl[l].y));
+        const int j = butterfly(li), par = half(li), k2 = li & 31, lo = j + 256 * par;
+        const float sg = par ? -1.f : 1.f;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();   // column `it` is in pre
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const float2 a = pre[j + q * 256], b = pre[j + (q + 16) * 256];
+            v[q] = make_float2(a.x + sg * b.x, a.y + sg * b.y);
+        }
+        if (par) turn32(v, -1);
+        dft16(v, -1);
+#pragma unroll
+        for (int q = 0; q < 16; ++q) buf[lidx(j * 32 + 2 * q + par)] = v[q];
+        lds_barrier();   // pre has been read by every wave
+        if (it + 1 < i1) prefetch(it + 1, span + (left == 1));
+#pragma unroll
+        for (int q = 0; q < 16; ++q) v[q] = buf[lidx(li + q * T)];
+        twiddle16_w(v, wm, -1);
+        dft16(v, -1);
+        lds_barrier();
+#pragma unroll
+        for (int q = 0; q < 16; ++q) buf[lidx((li - k2) * 16 + k2 + q * 32)] = v[q];
+        lds_barrier();
+#pragma unroll
+        for (int q = 0; q < 16; ++q) v[q] = buf[lidx(li + q * T)];
+        twiddle16_w(v, wl, -1);
+        dft16(v, -1);
+        if (f == 0) {   // the packed theta-DC and -Nyquist columns (k_cols_stream)
+            lds_barrier();
+#pragma unroll
+            for (int q = 0; q < 16; ++q) buf[lidx(li + q * T)] = v[q];
+            lds_barrier();
+            const float2* fzh = fzT + (size_t)h * M;
+#pragma unroll
+            for (int q = 0; q < 16; ++q) {
+                const int k = li + q * T;
+                const float2 A = v[q], Bc = cconj(buf[lidx(k == 0 ? 0 : M - k)]);
+                const float2 D = make_float2(0.5f * (A.x + Bc.x), 0.5f * (A.y + Bc.y));
+                const float2 Q = make_float2(0.5f * (A.y - Bc.y), -0.5f * (A.x - Bc.x));
+                v[q] = cadd(cmul(D, kz[q]), rot90(cmul(Q, fzval(fzh, k, rp.conj)), 1));
+                if (q % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+            lds_barrier();
+        } else {
+#pragma unroll
+            for (int q = 0; q < 16; ++q) v[q] = cmul(v[q], kz[q]);
+        }
+        // (a lane writes the slots that it alone has read: no barrier before)
+        dft16(v, +1);
+        twiddle16_w(v, wl, +1);
+#pragma unroll
+        for (int q = 0; q < 16; ++q) buf[lidx(li + q * T)] = v[q];
+        lds_barrier();
+#pragma unroll
+        for (int q = 0; q < 16; ++q) v[q] = buf[lidx((li - k2) * 16 + k2 + q * 32)];
+        dft16(v, +1);
+        twiddle16_w(v, wm, +1);
+        lds_barrier();
+#pragma unroll
+        for (int q = 0; q < 16; ++q) buf[lidx(li + q * T)] = v[q];
+        lds_barrier();
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const float2 a = buf[lidx(j * 32 + q)], b = buf[lidx(j * 32 + 16 + q)];
+            v[q] = make_float2(a.x + sg * b.x, a.y + sg * b.y);
+        }
+        if (par) turn32(v, +1);
+        dft16(v, +1);
+        const unsigned sm = span == 0 ? smask[0] : span == 1 ? smask[1] : smask[2];
+        float2* col = column(it);
+        const unsigned lane = (unsigned)lo * 8u;
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+            if (sm & (1u << q)) st_at_nt(col, lane + (unsigned)(q * T) * 8u, v[q]);
+        if (--left == 0) {
+            ++span;
+            left = rp.nz;
+        }
+        lds_barrier();
+    }
+}
+
 // Barrier over the lanes that share a row.  When a row fits in one wave
 // (h <= 1024) its lanes execute together and a wave's LDS operations complete
 // in issue order, so a wave-scope fence pair around a compiler-level wave
@@ -2103,7 +2261,7 @@ bool launch_rows_inv_polar(const RowPass& rp0, const PolarOut& po, hipStream_t s
 
 // middle radix of M = 16 * MID * 16, or 0 when the register kernel does not apply
 static int cols16_mid(int M) {
-    if (M < 256 || M > 4096 || (M & (M - 1))) return 0;
+    if (M < 256 || M > 8192 || (M & (M - 1))) return 0;
     return M / 256;
 }
 
@@ -2127,6 +2285,14 @@ void launch_cols(const RowPass& rp0, const FftPlan& planM, const float2* twM, co
             case 2: cols_stream<2>(rp0, twM, fzT, s); break;
             case 4: cols_stream<4>(rp0, twM, fzT, s); break;
             case 8: cols_stream<8>(rp0, twM, fzT, s); break;
+            case 32: {
+                // (one block per compute unit)
+                int items = std::min(3 * rp0.zgroup, 3 * rp0.nz);
+                while (items > 1 && (long long)rp0.h * ((3 * rp0.nz + items - 1) / items) < 1024) items = (items + 1) / 2;
+                hipLaunchKernelGGL(k_cols_stream32, dim3(rp0.h * ((3 * rp0.nz + items - 1) / items)), dim3(512), 0, s, rp0,
+                                   items, twM, fzT);
+                break;
+            }
             default: cols_stream<16>(rp0, twM, fzT, s); break;
         }
         return;

@@ -43,3 +43,31 @@ def test_column_pass_matches_oracle(torch_cuda, N0, P0, ns, check):
     ea = rel(fo.cpu().numpy()[at], mirror.adj(tab, R[at]))
     print("N0 %d: fwd %.2e adj %.2e" % (N0, ef, ea), flush=True)
     assert ef <= 1e-6 and ea <= 1e-6
+
+
+@pytest.mark.parametrize("ns", [1, 2])
+def test_column_pass_8192_matches_mixed_radix(torch_cuda, ns):
+    """rho 8192 (32 x 16 x 16): against the mixed-radix kernels (family 0), 3
+    and 6 columns per frequency; the same input and bound."""
+    torch = torch_cuda
+    print("case 4096", ns, flush=True)
+    N0, P0 = 4096, 48
+    g = torch.Generator(device="cuda").manual_seed(ns)
+    f = 1.0 + 0.1 * torch.randn((ns, N0, N0), device="cuda", generator=g)
+    R = 1.0 + 0.1 * torch.randn((ns, P0, N0), device="cuda", generator=g)
+    lp = lpTransform(N0, P0, ns, "none", N0 / 2, "cubic")
+    lp.precompute(1)
+    lp.initcmem(1, 0)
+    out = []
+    for family in (2, 0):
+        lp.clphandle[0].set_tuning(4, family)
+        a, b = torch.full_like(R, float("nan")), torch.full_like(f, float("nan"))
+        lp.fwdp(a, f, 0)
+        lp.adjp(b, R, 0)
+        torch.cuda.synchronize()
+        out.append((a, b))
+    lp.close()
+    for x, y in zip(*out):
+        e = float((x.double() - y.double()).norm() / y.double().norm())
+        print("rel %.1e" % e, flush=True)
+        assert e <= 1e-6
