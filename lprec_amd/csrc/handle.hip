@@ -1054,10 +1054,19 @@ void rtc_build(lp_handle* h) {
         const int waves = (int)(160 * 1024 / lds) * (nt / 64);
         return std::to_string(std::max(2, std::min(4, waves / 4)));
     };
-    // index arithmetic redone per slice; up to 256 points there are registers
-    // to hold it (and the twiddles, whose latency short kernels would expose):
-    // N = 256, 4 slices 104 -> 101 us; N = 528 the other way, 172 -> 586 us (spills)
-    auto opaque = [&](int M) { return M > 256 && (h->rtc_cols_var & 2) != 0; };
+    // index arithmetic redone per slice; up to 256 points and 8 elements per
+    // lane there are registers to hold it (and the twiddles, whose latency short
+    // kernels would expose): N = 256, 4 slices 104 -> 101 us.  Otherwise it
+    // spills: N = 528 172 -> 586 us, N = 432, 11 slices (216 points, radix 18)
+    // row passes 102 / 139 us against 26 / 23
+    auto opaque = [&](const CtPlan& p, int M, int NL) {
+        if (!(h->rtc_cols_var & 2)) return false;
+        for (int r : p.radix) {
+            const int items = (NL * (M / r) + p.nt - 1) / p.nt;
+            if (M > 256 || r >= 17 || items * r > 8) return true;
+        }
+        return false;
+    };
     // only the passes this handle runs (slot: 0 rows fwd, 1 rows inv, 2 cols,
     // 3 filtered sinogram pair)
     std::vector<std::string> names;
@@ -1088,7 +1097,7 @@ void rtc_build(lp_handle* h) {
             while (ls % 32 != (32 / R) % 32) ++ls;
             rnt = p.nt;
             const std::string args = std::to_string(h->h) + ", " + std::to_string(R) + ", " + std::to_string(ls) + ", " +
-                                     std::to_string(rnt) + ", " + wpe((size_t)R * ls * sizeof(float2), rnt) + (opaque(h->h) ? ", 1" : ", 0") + radix_args(p);
+                                     std::to_string(rnt) + ", " + wpe((size_t)R * ls * sizeof(float2), rnt) + (opaque(p, h->h, R) ? ", 1" : ", 0") + radix_args(p);
             name(0, "k_rows_fwd_ct<" + args);
             name(1, "k_rows_inv_ct<" + args);
         } else {
@@ -1102,7 +1111,7 @@ void rtc_build(lp_handle* h) {
             cnt = p.nt;
             name(2, "k_cols_ct<" + std::to_string(h->Nr) + ", " + std::to_string(cnt) + ", " +
                         wpe(ct_slots(p, h->Nr) * sizeof(float2), cnt) + ", " +
-                        (opaque(h->Nr) ? "2" : "0") + radix_args(p));
+                        (opaque(p, h->Nr, 1) ? "2" : "0") + radix_args(p));
         } else {
             err = "no plan for the column length";
         }
