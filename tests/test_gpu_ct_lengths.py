@@ -54,6 +54,7 @@ def _run(lp, f, R, torch):
     (304, 120, 1, "none", 152, "cubic"),     # 19
     (496, 180, 1, "ramp", 248, "cubic"),     # 31: 16 outputs, exactly one tile
     (526, 180, 2, "none", 263.4, "cubic"),   # N = 528: register radices 22 and 24
+    (417, 120, 11, "parzen", 208.5, "cubic"),# N = 432: 216 points as 18 x 12, slices in turn
     (592, 200, 1, "none", 296, "linear"),    # 37: 19 outputs, two tiles
     (752, 240, 1, "parzen", 376, "cubic"),   # 47: 24 terms, six full steps
 ])
