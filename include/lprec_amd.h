@@ -176,6 +176,13 @@ int lp_profile_read(lp_handle* h, int which, float* ms, int* ncalls);
  * `bytes` must not exceed the buffer; returns LP_ERR_ARG otherwise. */
 int lp_debug_stop(lp_handle* h, int stage);
 int lp_debug_copy(lp_handle* h, int which, void* dst, size_t bytes);
+/* The row, column and (filter != 0) filtered sinogram passes that a handle of
+ * padded size N, P0 angles and Ns slices compiles at run time, as template
+ * instantiations of rtc_kernels.hpp, one per line in names[cap] (truncated to
+ * fit): cols_threads as tuning key 11, lds = bytes of LDS a block may hold.
+ * Host arithmetic only, no device needed.  Returns the bytes that all of them
+ * take with the final 0, or LP_ERR_ARG. */
+int lp_debug_rtc_names(int N, int P0, int Ns, int filter, int cols_threads, int lds, char* names, int cap);
 
 #ifdef __cplusplus
 }

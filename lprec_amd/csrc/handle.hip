@@ -62,6 +62,9 @@ FftPlan make_plan(int M) {
 
 }  // namespace
 
+// default variant of the compiled passes (lp_handle::rtc_cols_var)
+constexpr int kRtcVar = 14;
+
 struct lp_handle {
     int device = 0;
     int N = 0, N0 = 0, Nt = 0, Nr = 0, P = 0, P0 = 0, Ns = 0, cor = 0, os = 1, h = 0;
@@ -89,7 +92,7 @@ struct lp_handle {
     int rtc_cols_req = 0;   // threads of the compiled column pass (0: automatic)
     // variant of the compiled passes: index arithmetic redone per slice (bit
     // 1), at least 4 waves per SIMD (bit 2); bits 0 and 3 have no effect
-    int rtc_cols_var = 14;
+    int rtc_cols_var = kRtcVar;
     bool rtc_tried = false;       // with the current settings ...
     bool rtc_pair_tried = false;  // ... and the filtered pair pass
     std::vector<hipModule_t> rtc_mods;
@@ -598,20 +601,14 @@ std::vector<float2> transpose_fz(const float* src, int Nr, int Nt) {
     return out;
 }
 
-// LDS line stride of the row passes (bank spreading is done by lidx())
-int row_ldm(const lp_handle* h, int R) {
-    (void)R;
-    return h->h;
-}
-
-int pick_rows(lp_handle* h) {
-    // log-polar rows per row-pass block: as many as the LDS and the FFT
-    // register budget allow, up to the tuned value
-    int R = h->R;
+// Log-polar rows of half length H per row-pass block: as many as the LDS and
+// the FFT register budget allow, up to R (Nr rows in all; the LDS line stride
+// is H, bank spreading is done by lidx())
+int pick_rows(int R, int H, int Nr, size_t lds_limit) {
     while (R > 1) {
-        size_t lds = lpk::rows_lds_bytes(row_ldm(h, R), R);
-        long long pts = (long long)R * h->h;
-        if (lds <= h->lds_limit && pts <= 32LL * 1024 && h->Nr % R == 0) break;
+        size_t lds = lpk::rows_lds_bytes(H, R);
+        long long pts = (long long)R * H;
+        if (lds <= lds_limit && pts <= 32LL * 1024 && Nr % R == 0) break;
         R /= 2;
     }
     return R;
@@ -916,7 +913,10 @@ double ct_radix_ops(int r) {
 // M = 4128 columns, 43 12 8 on 192 threads 2.60 ms, on 256 2.99, on 384 3.5,
 // 43 8 4 3 on 192 2.93; rows of h = 1032, 43 24 on 512 threads 1.41 inverse,
 // on 384 2.0; 320 or 576 threads (uneven waves per SIMD) 1.5-2 times slower.
-CtPlan ct_plan(int M, int NL, size_t lds_line, size_t lds_limit, double blocks, int force_nt) {
+// lds_line: LDS of a line, for the blocks that share a CU; lds(odd): all
+// that a block holds when the first radix is odd or even, for the limit.
+template <class Lds>
+CtPlan ct_plan(int M, int NL, size_t lds_line, Lds lds, size_t lds_limit, double blocks, int force_nt) {
     CtPlan best;
     if (NL * lds_line > lds_limit) return best;
     std::vector<int> primes;
@@ -935,6 +935,8 @@ CtPlan ct_plan(int M, int NL, size_t lds_line, size_t lds_limit, double blocks, 
     std::vector<int> cur;
     auto consider = [&](int nt) {
         if (nt > 64 && nt * 4 > NL * M) return;
+        const bool odd = !big.empty() || std::any_of(cur.begin(), cur.end(), [](int r) { return r & 1; });
+        if (lds(odd) > lds_limit) return;
         const double waves = nt / 64.0;
         // staging and stores (in the row passes also the R2C step, transposed access)
         double cost = (double)NL * M / nt * (NL > 1 ? 30 : 10);
@@ -997,8 +999,25 @@ std::string radix_args(const CtPlan& p) {
     return r;
 }
 
-// LDS slots of a line of M points under the plan (slots() of fft_ct.hpp)
-int ct_slots(const CtPlan& p, int M) { return (p.radix[0] & 1) ? M : M + (M >> 4) + 1; }
+// LDS slots of a line of M points whose first radix is odd or even (slots()
+// of fft_ct.hpp)
+int ct_slots(bool odd, int M) { return odd ? M : M + (M >> 4) + 1; }
+
+// Slots between the R lines of a row block (LS of rtc_kernels.hpp)
+int ct_row_stride(bool odd, int H, int R) {
+    int ls = ct_slots(odd, H);
+    while (ls % 32 != (32 / R) % 32) ++ls;
+    return ls;
+}
+
+// LDS of a block: all that the kernels of rtc_kernels.hpp declare, and in the
+// row passes what the compiler adds (256 bytes for __syncthreads_or, padding
+// between the arrays).  A kernel above the limit does not compile.
+size_t ct_rows_lds(bool odd, int H, int R) {
+    return ((size_t)R * ct_row_stride(odd, H, R) + H / 2 + 1 + R) * sizeof(float2) + 256 + 3 * 16;
+}
+size_t ct_cols_lds(bool odd, int M) { return (size_t)(ct_slots(odd, M) + 127) / 128 * 128 * sizeof(float2); }
+size_t ct_pair_lds(bool odd, int M) { return (size_t)ct_slots(odd, M) * sizeof(float2); }
 
 // Weights of the matrix-core stages (mfma_stage of fft_ct.hpp) of the prime
 // factors >= 17 of M, largest first: per tile of 16 outputs p and step of 4
@@ -1025,6 +1044,110 @@ std::vector<float> ct_weights(int M) {
     return w;
 }
 
+// The compiled passes of a handle: their instantiations, what each one is
+// (slot: 0 rows fwd, 1 rows inv, 2 cols, 3 filtered sinogram pair) and their
+// launch shapes.
+struct RtcPlan {
+    std::vector<std::string> names;
+    std::vector<int> slot;
+    int R = 0, rows_nt = 0, cols_nt = 0, pair_nt = 0;
+    std::string err;
+};
+
+// What the plan of a handle depends on: the padded grid, its angles and
+// slices, the most rows per block, the settings of the compiled passes and
+// the LDS of a block.
+struct RtcShape {
+    int N, P0, Ns, R, cols_nt, var;
+    size_t lds_limit;
+};
+
+RtcPlan rtc_plan(const RtcShape& s, bool rows, bool cols, bool pair) {
+    const int H = s.N / 2, Nr = 2 * s.N;
+    RtcPlan out;
+    // waves per SIMD the registers are budgeted for: what the blocks' LDS lets
+    // a CU hold, up to 4 (128 registers)
+    auto wpe = [&](size_t lds, int nt) {
+        if (!(s.var & 4)) return std::string("2");
+        const int waves = (int)(160 * 1024 / lds) * (nt / 64);
+        return std::to_string(std::max(2, std::min(4, waves / 4)));
+    };
+    // index arithmetic redone per slice; up to 256 points and 8 elements per
+    // lane there are registers to hold it (and the twiddles, whose latency short
+    // kernels would expose): N = 256, 4 slices 104 -> 101 us.  Otherwise it
+    // spills: N = 528 172 -> 586 us, N = 432, 11 slices (216 points, radix 18)
+    // row passes 102 / 139 us against 26 / 23
+    auto opaque = [&](const CtPlan& p, int M, int NL) {
+        if (!(s.var & 2)) return false;
+        for (int r : p.radix) {
+            const int items = (NL * (M / r) + p.nt - 1) / p.nt;
+            if (M > 256 || r >= 17 || items * r > 8) return true;
+        }
+        return false;
+    };
+    auto name = [&](int k, const std::string& n) {
+        out.names.push_back("lpct::" + n + ">");
+        out.slot.push_back(k);
+    };
+    if (rows) {
+        // rows per block: 16 give 128-byte segments of the transposed spectra
+        // (8 and 4: 64 and 32 bytes), fewer give a small batch more blocks
+        CtPlan p;
+        int R = 0;
+        const size_t line = (size_t)(H + (H >> 4) + 32) * sizeof(float2);   // padded, with the row offset
+        for (int r = std::min(s.R, 16); r >= 1; r /= 2) {
+            if (Nr % r || (p.ok() && r < 4)) continue;
+            CtPlan q = ct_plan(H, r, line, [&](bool odd) { return ct_rows_lds(odd, H, r); }, s.lds_limit,
+                               3.0 * s.Ns * (Nr / r), 0);
+            if (3LL * s.Ns * Nr / r * q.nt > 256 * 1024) q.cost *= r >= 16 ? 1.0 : r >= 8 ? 1.04 : r >= 4 ? 1.25 : 2.0;
+            if (q.ok() && (!p.ok() || q.cost < p.cost)) {
+                p = q;
+                R = r;
+            }
+        }
+        if (p.ok()) {
+            const bool odd = p.radix[0] & 1;
+            const std::string args = std::to_string(H) + ", " + std::to_string(R) + ", " +
+                                     std::to_string(ct_row_stride(odd, H, R)) + ", " + std::to_string(p.nt) + ", " +
+                                     wpe((size_t)R * ct_row_stride(odd, H, R) * sizeof(float2), p.nt) + (opaque(p, H, R) ? ", 1" : ", 0") + radix_args(p);
+            name(0, "k_rows_fwd_ct<" + args);
+            name(1, "k_rows_inv_ct<" + args);
+            out.R = R;
+            out.rows_nt = p.nt;
+        } else {
+            out.err = "no plan for the row length";
+        }
+    }
+    if (cols) {
+        const CtPlan p = ct_plan(Nr, 1, (size_t)(Nr + (Nr >> 4) + 1) * sizeof(float2),
+                                 [&](bool odd) { return ct_cols_lds(odd, Nr); }, s.lds_limit, 3.0 * s.Ns * H, s.cols_nt);
+        if (p.ok()) {
+            out.cols_nt = p.nt;
+            name(2, "k_cols_ct<" + std::to_string(Nr) + ", " + std::to_string(p.nt) + ", " +
+                        wpe(ct_slots(p.radix[0] & 1, Nr) * sizeof(float2), p.nt) + ", " + (opaque(p, Nr, 1) ? "2" : "0") + radix_args(p));
+        } else {
+            out.err = "no plan for the column length";
+        }
+    }
+    if (pair) {
+        const int M = 2 * s.N;
+        const CtPlan p = ct_plan(M, 1, (size_t)(M + (M >> 4) + 1) * sizeof(float2),
+                                 [&](bool odd) { return ct_pair_lds(odd, M); }, s.lds_limit, 0.5 * s.Ns * s.P0, 0);
+        if (p.ok()) {
+            out.pair_nt = p.nt;
+            name(3, "k_sino_rows_pair_ct<" + std::to_string(s.N) + ", " + std::to_string(p.nt) + ", " +
+                        wpe(ct_slots(p.radix[0] & 1, M) * sizeof(float2), p.nt) + radix_args(p));
+        } else {
+            out.err = "no plan for the filter length";
+        }
+    }
+    return out;
+}
+
+// lengths that no register kernel covers (rows of H points, columns of Nr)
+bool rtc_rows_needed(int H) { return !pow2_in(H, 256, 4096); }
+bool rtc_cols_needed(int Nr) { return !pow2_in(Nr, 256, 8192); }
+
 void rtc_build(lp_handle* h) {
     if (!h->rtc_mode) return;
     if (!h->rtc_tried) {
@@ -1033,7 +1156,8 @@ void rtc_build(lp_handle* h) {
         h->rtc_fn[0] = h->rtc_fn[1] = h->rtc_fn[2] = h->rtc_fn[3] = nullptr;
         h->rtc_pair_tried = false;
     }
-    const bool rows = !h->rtc_tried && !pow2_in(h->h, 256, 4096), cols = !h->rtc_tried && !pow2_in(h->Nr, 256, 8192);
+    // only the passes this handle runs
+    const bool rows = !h->rtc_tried && rtc_rows_needed(h->h), cols = !h->rtc_tried && rtc_cols_needed(h->Nr);
     // the filtered pair pass has no register kernel at any length; when the
     // filter comes after the first build (lp_init_adj after lp_init_fwd), it
     // is a module of its own
@@ -1047,126 +1171,47 @@ void rtc_build(lp_handle* h) {
     if (hipGetDeviceProperties(&prop, h->device) != hipSuccess) return;
     std::string arch(prop.gcnArchName);
     arch = arch.substr(0, arch.find(':'));
-    // waves per SIMD the registers are budgeted for: what the blocks' LDS lets
-    // a CU hold, up to 4 (128 registers)
-    auto wpe = [&](size_t lds, int nt) {
-        if (!(h->rtc_cols_var & 4)) return std::string("2");
-        const int waves = (int)(160 * 1024 / lds) * (nt / 64);
-        return std::to_string(std::max(2, std::min(4, waves / 4)));
-    };
-    // index arithmetic redone per slice; up to 256 points and 8 elements per
-    // lane there are registers to hold it (and the twiddles, whose latency short
-    // kernels would expose): N = 256, 4 slices 104 -> 101 us.  Otherwise it
-    // spills: N = 528 172 -> 586 us, N = 432, 11 slices (216 points, radix 18)
-    // row passes 102 / 139 us against 26 / 23
-    auto opaque = [&](const CtPlan& p, int M, int NL) {
-        if (!(h->rtc_cols_var & 2)) return false;
-        for (int r : p.radix) {
-            const int items = (NL * (M / r) + p.nt - 1) / p.nt;
-            if (M > 256 || r >= 17 || items * r > 8) return true;
-        }
-        return false;
-    };
-    // only the passes this handle runs (slot: 0 rows fwd, 1 rows inv, 2 cols,
-    // 3 filtered sinogram pair)
-    std::vector<std::string> names;
-    std::vector<int> slot;
-    int R = 0, rnt = 0, cnt = 0, pnt = 0;
-    std::string err;
-    auto name = [&](int k, const std::string& n) {
-        names.push_back("lpct::" + n + ">");
-        slot.push_back(k);
-    };
-    if (rows) {
-        // rows per block: 16 give 128-byte segments of the transposed spectra
-        // (8 and 4: 64 and 32 bytes), fewer give a small batch more blocks
-        CtPlan p;
-        int ls = 0;
-        const size_t line = (size_t)(h->h + (h->h >> 4) + 32) * sizeof(float2);   // padded, with the row offset
-        for (int r = std::min(h->R, 16); r >= 1; r /= 2) {
-            if (h->Nr % r || (p.ok() && r < 4)) continue;
-            CtPlan q = ct_plan(h->h, r, line, h->lds_limit, 3.0 * h->Ns * (h->Nr / r), 0);
-            if (3LL * h->Ns * h->Nr / r * q.nt > 256 * 1024) q.cost *= r >= 16 ? 1.0 : r >= 8 ? 1.04 : r >= 4 ? 1.25 : 2.0;
-            if (q.ok() && (!p.ok() || q.cost < p.cost)) {
-                p = q;
-                R = r;
-            }
-        }
-        if (p.ok()) {
-            ls = ct_slots(p, h->h);
-            while (ls % 32 != (32 / R) % 32) ++ls;
-            rnt = p.nt;
-            const std::string args = std::to_string(h->h) + ", " + std::to_string(R) + ", " + std::to_string(ls) + ", " +
-                                     std::to_string(rnt) + ", " + wpe((size_t)R * ls * sizeof(float2), rnt) + (opaque(p, h->h, R) ? ", 1" : ", 0") + radix_args(p);
-            name(0, "k_rows_fwd_ct<" + args);
-            name(1, "k_rows_inv_ct<" + args);
-        } else {
-            err = "no plan for the row length";
-        }
-    }
-    if (cols) {
-        const CtPlan p = ct_plan(h->Nr, 1, (size_t)(h->Nr + (h->Nr >> 4) + 1) * sizeof(float2), h->lds_limit,
-                                 3.0 * h->Ns * h->h, h->rtc_cols_req);
-        if (p.ok()) {
-            cnt = p.nt;
-            name(2, "k_cols_ct<" + std::to_string(h->Nr) + ", " + std::to_string(cnt) + ", " +
-                        wpe(ct_slots(p, h->Nr) * sizeof(float2), cnt) + ", " +
-                        (opaque(p, h->Nr, 1) ? "2" : "0") + radix_args(p));
-        } else {
-            err = "no plan for the column length";
-        }
-    }
-    if (pair) {
-        const CtPlan p = ct_plan(2 * h->N, 1, (size_t)(2 * h->N + (2 * h->N >> 4) + 1) * sizeof(float2), h->lds_limit,
-                                 0.5 * h->Ns * h->P0, 0);
-        if (p.ok()) {
-            pnt = p.nt;
-            name(3, "k_sino_rows_pair_ct<" + std::to_string(h->N) + ", " + std::to_string(pnt) + ", " +
-                        wpe(ct_slots(p, 2 * h->N) * sizeof(float2), pnt) + radix_args(p));
-        } else {
-            err = "no plan for the filter length";
-        }
-    }
+    RtcPlan p = rtc_plan({h->N, h->P0, h->Ns, h->R, h->rtc_cols_req, h->rtc_cols_var, h->lds_limit}, rows, cols, pair);
     if (!h->d_wodd) {
         // h, Nr and 2N are N times powers of two: they share their large primes
         const std::vector<float> w = ct_weights(h->N);
         if (!w.empty() && h->upload(&h->d_wodd, w)) return;
     }
     std::shared_ptr<RtcCode> code;
-    if (!names.empty()) code = rtc_compile(arch, names, err);
+    if (!p.names.empty()) code = rtc_compile(arch, p.names, p.err);
     hipModule_t mod = nullptr;
     if (code && hipModuleLoadData(&mod, code->code.data()) != hipSuccess) {
         (void)hipGetLastError();
-        err = "hipModuleLoadData failed";
+        p.err = "hipModuleLoadData failed";
         mod = nullptr;
     }
     void* fn[4] = {nullptr, nullptr, nullptr, nullptr};
-    for (size_t i = 0; mod && i < names.size(); ++i) {
+    for (size_t i = 0; mod && i < p.names.size(); ++i) {
         hipFunction_t f = nullptr;
         if (hipModuleGetFunction(&f, mod, code->lowered[i].c_str()) != hipSuccess) {
             (void)hipGetLastError();
-            err = "hipModuleGetFunction failed for " + names[i];
+            p.err = "hipModuleGetFunction failed for " + p.names[i];
             (void)hipModuleUnload(mod);
             mod = nullptr;
             break;
         }
-        fn[slot[i]] = (void*)f;
+        fn[p.slot[i]] = (void*)f;
     }
     if (!mod) {
-        if (verbose) std::fprintf(stderr, "lprec_amd: run-time compiled passes unavailable (%s)\n", err.c_str());
+        if (verbose) std::fprintf(stderr, "lprec_amd: run-time compiled passes unavailable (%s)\n", p.err.c_str());
         return;
     }
     h->rtc_mods.push_back(mod);
     for (int i = 0; i < 4; ++i)
         if (fn[i]) h->rtc_fn[i] = fn[i];
     if (rows) {
-        h->rtc_R = R;
-        h->rtc_rows_nt = rnt;
+        h->rtc_R = p.R;
+        h->rtc_rows_nt = p.rows_nt;
     }
-    if (cols) h->rtc_cols_nt = cnt;
-    if (pair) h->rtc_pair_nt = pnt;
+    if (cols) h->rtc_cols_nt = p.cols_nt;
+    if (pair) h->rtc_pair_nt = p.pair_nt;
     if (verbose)
-        for (const auto& n : names) std::fprintf(stderr, "lprec_amd: run-time compiled pass: %s\n", n.c_str());
+        for (const auto& n : p.names) std::fprintf(stderr, "lprec_amd: run-time compiled pass: %s\n", n.c_str());
 }
 
 }  // namespace
@@ -1204,7 +1249,7 @@ int lp_create(const float* g, int device, lp_handle** out) {
     if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) == hipSuccess && lds > 0)
         h->lds_limit = (size_t)lds;
     h->R = 16;
-    h->R = pick_rows(h.get());
+    h->R = pick_rows(h->R, h->h, h->Nr, h->lds_limit);
     try {
         h->plan_h = make_plan(h->h);
         h->plan_N = make_plan(h->N);
@@ -1601,7 +1646,7 @@ static void scatter_to(lp_handle* h, lpk::Scatter g, const lpk::GTile* tiles, in
 static lpk::RowPass row_pass(lp_handle* h, int nz) {
     lpk::RowPass rp;
     rp.Ntheta = h->Nt; rp.Nrho = h->Nr; rp.h = h->h; rp.R = h->R;
-    rp.ldm = row_ldm(h, h->R);
+    rp.ldm = h->h;
     rp.nz = nz;
     rp.zgroup = std::max(1, std::min(h->zgroup, nz));
     rp.planh = h->plan_h;
@@ -1976,7 +2021,7 @@ int lp_set_tuning(lp_handle* h, int key, int value) {
             if (value < 1 || value > 16 || (value & (value - 1))) return h->fail(LP_ERR_ARG, "rows per block must be a power of two in [1, 16]");
             int old = h->R;
             h->R = value;
-            int r = pick_rows(h);
+            int r = pick_rows(h->R, h->h, h->Nr, h->lds_limit);
             if (r != value) { h->R = old; return h->fail(LP_ERR_ARG, "rows per block exceeds the LDS or FFT budget"); }
             return LP_OK;
         }
@@ -2114,6 +2159,20 @@ int lp_debug_copy(lp_handle* h, int which, void* dst, size_t bytes) {
     if (hipDeviceSynchronize() != hipSuccess || hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost) != hipSuccess)
         return h->fail(LP_ERR_DEVICE, "device to host copy failed");
     return LP_OK;
+}
+
+int lp_debug_rtc_names(int N, int P0, int Ns, int filter, int cols_threads, int lds, char* names, int cap) {
+    if (N < 16 || N % 16 || P0 < 1 || Ns < 1 || lds < 1 || cap < 0 || (cap && !names)) return LP_ERR_ARG;
+    const int R = pick_rows(16, N / 2, 2 * N, (size_t)lds);
+    const RtcPlan p = rtc_plan({N, P0, Ns, R, cols_threads, kRtcVar, (size_t)lds},
+                               rtc_rows_needed(N / 2), rtc_cols_needed(2 * N), filter != 0);
+    std::string all;
+    for (const auto& n : p.names) all += n + "\n";
+    if (cap) {
+        std::strncpy(names, all.c_str(), (size_t)cap - 1);
+        names[cap - 1] = 0;
+    }
+    return (int)all.size() + 1;
 }
 
 int lp_get_tuning(const lp_handle* h, int key, int* value) {
