@@ -183,6 +183,9 @@ int lp_debug_copy(lp_handle* h, int which, void* dst, size_t bytes);
  * Host arithmetic only, no device needed.  Returns the bytes that all of them
  * take with the final 0, or LP_ERR_ARG. */
 int lp_debug_rtc_names(int N, int P0, int Ns, int filter, int cols_threads, int lds, char* names, int cap);
+/* Compiles such passes (at most 32, one per line) for gfx950 as a handle does;
+ * bit i of *compiled is set when pass i has code.  No device needed. */
+int lp_debug_rtc_compile(const char* names, unsigned* compiled);
 
 #ifdef __cplusplus
 }

@@ -811,7 +811,7 @@ int polar_transpose_tables(lp_handle* h, const std::vector<float2>& p2lp, const 
 // passes with every size a template argument) for this handle's lengths and
 // radix sequences with hipRTC, once per process and set of lengths, and loads
 // the code object on the handle's device.  Failure is not an error: the
-// generic kernels stay in use (LPREC_AMD_VERBOSE=1 prints why).
+// generic kernel stays in use for that pass (LPREC_AMD_VERBOSE=1 prints why).
 
 // directory of the device sources next to the shared library
 std::string csrc_dir() {
@@ -877,6 +877,25 @@ std::shared_ptr<RtcCode> rtc_compile(const std::string& arch, const std::vector<
     }
     hiprtcDestroyProgram(&prog);
     g_rtc_cache[key] = out;
+    return out;
+}
+
+// The programs of the named passes: one for all of them (they share the time
+// to read the headers: 1.85 s for the four of N = 2064, 2.25 s one by one), or,
+// when that does not compile, one for each pass that does.
+struct RtcProgram {
+    std::shared_ptr<RtcCode> code;
+    std::vector<size_t> at;   // the passes in it
+};
+std::vector<RtcProgram> rtc_programs(const std::string& arch, const std::vector<std::string>& names, std::string& err) {
+    std::vector<RtcProgram> out;
+    if (auto code = rtc_compile(arch, names, err)) {
+        out.push_back({code, {}});
+        for (size_t i = 0; i < names.size(); ++i) out[0].at.push_back(i);
+        return out;
+    }
+    for (size_t i = 0; names.size() > 1 && i < names.size(); ++i)
+        if (auto code = rtc_compile(arch, {names[i]}, err)) out.push_back({code, {i}});
     return out;
 }
 
@@ -1177,41 +1196,35 @@ void rtc_build(lp_handle* h) {
         const std::vector<float> w = ct_weights(h->N);
         if (!w.empty() && h->upload(&h->d_wodd, w)) return;
     }
-    std::shared_ptr<RtcCode> code;
-    if (!p.names.empty()) code = rtc_compile(arch, p.names, p.err);
-    hipModule_t mod = nullptr;
-    if (code && hipModuleLoadData(&mod, code->code.data()) != hipSuccess) {
-        (void)hipGetLastError();
-        p.err = "hipModuleLoadData failed";
-        mod = nullptr;
-    }
-    void* fn[4] = {nullptr, nullptr, nullptr, nullptr};
-    for (size_t i = 0; mod && i < p.names.size(); ++i) {
-        hipFunction_t f = nullptr;
-        if (hipModuleGetFunction(&f, mod, code->lowered[i].c_str()) != hipSuccess) {
+    const std::vector<RtcProgram> programs = p.names.empty() ? std::vector<RtcProgram>() : rtc_programs(arch, p.names, p.err);
+    for (const RtcProgram& g : programs) {
+        hipModule_t mod = nullptr;
+        if (hipModuleLoadData(&mod, g.code->code.data()) != hipSuccess) {
             (void)hipGetLastError();
-            p.err = "hipModuleGetFunction failed for " + p.names[i];
-            (void)hipModuleUnload(mod);
-            mod = nullptr;
-            break;
+            p.err = "hipModuleLoadData failed";
+            continue;
         }
-        fn[p.slot[i]] = (void*)f;
+        h->rtc_mods.push_back(mod);
+        for (size_t i = 0; i < g.at.size(); ++i) {
+            const std::string& n = p.names[g.at[i]];
+            hipFunction_t f = nullptr;
+            if (hipModuleGetFunction(&f, mod, g.code->lowered[i].c_str()) != hipSuccess) {
+                (void)hipGetLastError();
+                p.err = "hipModuleGetFunction failed for " + n;
+                continue;
+            }
+            h->rtc_fn[p.slot[g.at[i]]] = (void*)f;
+            if (verbose) std::fprintf(stderr, "lprec_amd: run-time compiled pass: %s\n", n.c_str());
+        }
     }
-    if (!mod) {
-        if (verbose) std::fprintf(stderr, "lprec_amd: run-time compiled passes unavailable (%s)\n", p.err.c_str());
-        return;
-    }
-    h->rtc_mods.push_back(mod);
-    for (int i = 0; i < 4; ++i)
-        if (fn[i]) h->rtc_fn[i] = fn[i];
     if (rows) {
         h->rtc_R = p.R;
         h->rtc_rows_nt = p.rows_nt;
     }
-    if (cols) h->rtc_cols_nt = p.cols_nt;
+    if (cols) h->rtc_cols_nt = h->rtc_fn[2] ? p.cols_nt : 0;
     if (pair) h->rtc_pair_nt = p.pair_nt;
-    if (verbose)
-        for (const auto& n : p.names) std::fprintf(stderr, "lprec_amd: run-time compiled pass: %s\n", n.c_str());
+    if (verbose && !p.err.empty())
+        std::fprintf(stderr, "lprec_amd: run-time compiled passes unavailable (%s)\n", p.err.c_str());
 }
 
 }  // namespace
@@ -2162,7 +2175,9 @@ int lp_debug_copy(lp_handle* h, int which, void* dst, size_t bytes) {
 }
 
 int lp_debug_rtc_names(int N, int P0, int Ns, int filter, int cols_threads, int lds, char* names, int cap) {
-    if (N < 16 || N % 16 || P0 < 1 || Ns < 1 || lds < 1 || cap < 0 || (cap && !names)) return LP_ERR_ARG;
+    if (N < 16 || N > 65536 || N % 16 || P0 < 1 || Ns < 1 || lds < 1 || cap < 0 || (cap && !names) ||
+        (cols_threads != 0 && cols_threads != 256 && cols_threads != 512 && cols_threads != 1024))
+        return LP_ERR_ARG;
     const int R = pick_rows(16, N / 2, 2 * N, (size_t)lds);
     const RtcPlan p = rtc_plan({N, P0, Ns, R, cols_threads, kRtcVar, (size_t)lds},
                                rtc_rows_needed(N / 2), rtc_cols_needed(2 * N), filter != 0);
@@ -2173,6 +2188,22 @@ int lp_debug_rtc_names(int N, int P0, int Ns, int filter, int cols_threads, int 
         names[cap - 1] = 0;
     }
     return (int)all.size() + 1;
+}
+
+int lp_debug_rtc_compile(const char* names, unsigned* compiled) {
+    if (!names || !compiled) return LP_ERR_ARG;
+    std::vector<std::string> list;
+    for (const char* p = names; *p;) {
+        const char* e = std::strchr(p, '\n');
+        list.emplace_back(p, e ? e : p + std::strlen(p));
+        p += list.back().size() + (e ? 1 : 0);
+    }
+    if (list.empty() || list.size() > 32) return LP_ERR_ARG;
+    *compiled = 0;
+    std::string err;
+    for (const RtcProgram& g : rtc_programs("gfx950", list, err))
+        for (size_t i : g.at) *compiled |= 1u << i;
+    return LP_OK;
 }
 
 int lp_get_tuning(const lp_handle* h, int key, int* value) {

@@ -91,3 +91,14 @@ def test_planned_passes_compile_for_gfx950(N, Ns):
     assert len(names) == 4, names   # rows there and back, columns, filtered pair
     log = _compile(names)
     assert log is None, log
+
+
+def test_a_pass_that_does_not_compile_leaves_the_others():
+    """Rows whose LDS is over the limit, beside columns and filter rows that compile."""
+    _hiprtc()
+    names = ["lpct::k_rows_fwd_ct<2304, 8, 2468, 768, 2, 1, 24, 12, 8>", "lpct::k_cols_ct<528, 64, 4, 2, 11, 12, 4>",
+             "lpct::k_sino_rows_pair_ct<264, 64, 4, 11, 12, 4>"]
+    assert _compile(names[:1]) is not None and _compile(names[1:]) is None
+    got = ctypes.c_uint()
+    assert _lib.load().lp_debug_rtc_compile("\n".join(names).encode(), ctypes.byref(got)) == 0
+    assert got.value == 0b110
