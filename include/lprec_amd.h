@@ -134,7 +134,7 @@ int lp_info(const lp_handle* h, int64_t* info);
  * row and column passes compiled at run time (hipRTC, at lp_init_fwd /
  * lp_init_adj) for transform lengths the radix-16 kernels do not cover (1,
  * the default; 0 = the generic mixed-radix kernels; reads back 1 only while
- * such passes are loaded), key 11 = threads per block of the compiled column
+ * every pass that the handle's lengths need is loaded), key 11 = threads per block of the compiled column
  * pass (256, 512 or 1024; 0 = automatic, the default; recompiles; reads back
  * the threads in use), key 12 = variant of the compiled passes, a 4-bit
  * mask (bit 1: their index arithmetic is redone per slice instead of held in

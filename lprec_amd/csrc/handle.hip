@@ -2219,7 +2219,12 @@ int lp_get_tuning(const lp_handle* h, int key, int* value) {
         case 7: *value = h->pt_ok ? h->polar_t : 0; return LP_OK;
         case 8: *value = h->staged; return LP_OK;
         case 9: *value = h->box_rule; return LP_OK;
-        case 10: *value = h->rtc_mode && !h->rtc_mods.empty() ? 1 : 0; return LP_OK;
+        case 10: {   // every pass that this handle's lengths need is loaded, and there is one
+            const bool rows = rtc_rows_needed(h->h), cols = rtc_cols_needed(h->Nr);
+            *value = h->rtc_mode && (rows || cols || h->has_filter) && (!rows || (h->rtc_fn[0] && h->rtc_fn[1])) &&
+                     (!cols || h->rtc_fn[2]) && (!h->has_filter || h->rtc_fn[3]);
+            return LP_OK;
+        }
         case 11: *value = h->rtc_cols_nt; return LP_OK;
         case 12: *value = h->rtc_cols_var; return LP_OK;
         case 13: *value = h->pzgroup; return LP_OK;

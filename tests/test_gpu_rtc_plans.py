@@ -1,7 +1,7 @@
-"""Compiled passes whose LDS is close to the limit: N = 4608 (rows of 2304
-points) against the generic kernels, adj with a filter.  Bound 2e-6, that of the
-other lengths against the generic kernels, whose odd radices form the powers of
-a root by recurrences."""
+"""What a handle's plan of the compiled passes does: rows whose LDS is close to the limit, and what the tuning
+keys of these passes read back and run.  N = 4608 (rows of 2304 points) against the generic kernels, adj with a
+filter: bound 2e-6, that of the other lengths against the generic kernels, whose odd radices form the powers of a root
+by recurrences."""
 import numpy as np
 import pytest
 
@@ -32,3 +32,17 @@ def test_rows_close_to_the_lds_limit(torch_cuda, ns):
     e = float((out[0] - out[1]).norm() / out[1].norm())
     print("compiled vs generic: %.2e" % e, flush=True)
     assert e <= 2e-6
+
+
+@pytest.mark.parametrize("N0,loaded", [
+    (2064, 1),
+    (6864, 0),   # no plan for the columns (13728 points: radix 13 alone has more butterflies than threads)
+])
+def test_key_10_tells_whether_every_pass_is_compiled(torch_cuda, N0, loaded):
+    print("case", N0, flush=True)
+    lp = lpTransform(N0, 48, 1, "none", N0 / 2, "cubic")
+    lp.precompute(0)
+    lp.initcmem(0, 0)
+    got = lp.clphandle[0].get_tuning(10)
+    lp.close()
+    assert got == loaded
