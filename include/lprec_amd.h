@@ -135,8 +135,9 @@ int lp_info(const lp_handle* h, int64_t* info);
  * lp_init_adj) for transform lengths the radix-16 kernels do not cover (1,
  * the default; 0 = the generic mixed-radix kernels; reads back 1 only while
  * every pass that the handle's lengths need is loaded), key 11 = threads per block of the compiled column
- * pass (256, 512 or 1024; 0 = automatic, the default; recompiles; reads back
- * the threads in use), key 12 = variant of the compiled passes, a 4-bit
+ * pass (256, 512 or 1024; 0 = automatic, the default, and where the length
+ * has no plan with that many; recompiles; reads back the threads in use, 0
+ * while no such pass is loaded), key 12 = variant of the compiled passes, a 4-bit
  * mask (bit 1: their index arithmetic is redone per slice instead of held in
  * registers, above 256 points; bit 2: registers budgeted for up to 4 waves
  * per SIMD, as many as the blocks' LDS admits, instead of 2; bits 0 and 3

@@ -934,8 +934,9 @@ double ct_radix_ops(int r) {
 // on 384 2.0; 320 or 576 threads (uneven waves per SIMD) 1.5-2 times slower.
 // lds_line: LDS of a line, for the blocks that share a CU; lds(odd): all
 // that a block holds when the first radix is odd or even, for the limit.
+// force_nt: threads per block (0: any); most: points per thread.
 template <class Lds>
-CtPlan ct_plan(int M, int NL, size_t lds_line, Lds lds, size_t lds_limit, double blocks, int force_nt) {
+CtPlan ct_plan(int M, int NL, size_t lds_line, Lds lds, size_t lds_limit, double blocks, int force_nt, int most = 24) {
     CtPlan best;
     if (NL * lds_line > lds_limit) return best;
     std::vector<int> primes;
@@ -953,7 +954,7 @@ CtPlan ct_plan(int M, int NL, size_t lds_line, Lds lds, size_t lds_limit, double
     std::sort(big.rbegin(), big.rend());
     std::vector<int> cur;
     auto consider = [&](int nt) {
-        if (nt > 64 && nt * 4 > NL * M) return;
+        if (!force_nt && nt > 64 && nt * 4 > NL * M) return;
         const bool odd = !big.empty() || std::any_of(cur.begin(), cur.end(), [](int r) { return r & 1; });
         if (lds(odd) > lds_limit) return;
         const double waves = nt / 64.0;
@@ -976,7 +977,7 @@ CtPlan ct_plan(int M, int NL, size_t lds_line, Lds lds, size_t lds_limit, double
         }
         for (int r : cur) {
             const long long items = (long long)NL * (M / r), ni = (items + nt - 1) / nt;
-            if (ni * r > 24) return;
+            if (ni * r > most) return;
             // above 16 points the butterfly's temporaries crowd the registers
             cost += (double)ni * r * ct_radix_ops(r) * (r > 16 ? 1.2 : 1.0) + 60 + 4 * waves;
         }
@@ -1138,8 +1139,14 @@ RtcPlan rtc_plan(const RtcShape& s, bool rows, bool cols, bool pair) {
         }
     }
     if (cols) {
-        const CtPlan p = ct_plan(Nr, 1, (size_t)(Nr + (Nr >> 4) + 1) * sizeof(float2),
-                                 [&](bool odd) { return ct_cols_lds(odd, Nr); }, s.lds_limit, 3.0 * s.Ns * H, s.cols_nt);
+        // a block size that was asked for is kept, also with threads to spare or
+        // up to 32 points (spilled) a thread; where even that leaves no plan,
+        // the automatic one
+        CtPlan p;
+        for (auto [nt, most] : {std::pair{s.cols_nt, 24}, std::pair{s.cols_nt, s.cols_nt ? 32 : 24}, std::pair{0, 24}})
+            if (!p.ok())
+                p = ct_plan(Nr, 1, (size_t)(Nr + (Nr >> 4) + 1) * sizeof(float2),
+                            [&](bool odd) { return ct_cols_lds(odd, Nr); }, s.lds_limit, 3.0 * s.Ns * H, nt, most);
         if (p.ok()) {
             out.cols_nt = p.nt;
             name(2, "k_cols_ct<" + std::to_string(Nr) + ", " + std::to_string(p.nt) + ", " +

@@ -46,3 +46,27 @@ def test_key_10_tells_whether_every_pass_is_compiled(torch_cuda, N0, loaded):
     got = lp.clphandle[0].get_tuning(10)
     lp.close()
     assert got == loaded
+
+
+@pytest.mark.parametrize("N0,ns", [(80, 2), (528, 8)])
+def test_threads_of_the_column_pass(torch_cuda, N0, ns):
+    """Key 11: every accepted count runs, reads back, and gives the automatic one's result (1e-6: the radices may
+    come in another order)."""
+    torch = torch_cuda
+    print("case", N0, ns, flush=True)
+    lp = lpTransform(N0, 60, ns, "none", N0 / 2, "cubic")
+    lp.precompute(0)
+    lp.initcmem(0, 0)
+    h = lp.clphandle[0]
+    R = torch.from_numpy(np.random.default_rng(N0).standard_normal((ns, 60, N0)).astype(np.float32)).cuda()
+    out = []
+    for threads in (0, 256, 512, 1024):
+        h.set_tuning(11, threads)
+        assert h.get_tuning(10) == 1 and (h.get_tuning(11) == threads or not threads)
+        f = torch.full((ns, N0, N0), float("nan"), device="cuda")
+        lp.adjp(f, R, 0)
+        torch.cuda.synchronize()
+        out.append(f.double())
+    lp.close()
+    for f in out[1:]:
+        assert float((f - out[0]).norm() / out[0].norm()) <= 1e-6

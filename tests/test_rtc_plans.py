@@ -102,3 +102,18 @@ def test_a_pass_that_does_not_compile_leaves_the_others():
     got = ctypes.c_uint()
     assert _lib.load().lp_debug_rtc_compile("\n".join(names).encode(), ctypes.byref(got)) == 0
     assert got.value == 0b110
+
+
+def test_threads_asked_for_keep_the_column_pass():
+    """Tuning key 11 at every length where it is accepted (32 points a thread): the columns have a plan, with that
+    many threads unless a thread would hold more than 16 points (a prime radix may not divide among them so)."""
+    for N in range(16, 4944, 16):
+        for threads in (256, 512, 1024):
+            if threads * 32 < 2 * N:
+                continue
+            names = [n for n in planned(N, N, 8, 0, threads) if "k_cols_ct" in n]
+            if not names:
+                assert N & (N - 1) == 0 and N >= 128, N   # the register kernels' lengths
+                continue
+            used = int(names[0].split(",")[1])
+            assert used == threads or 2 * N > 16 * threads, names
