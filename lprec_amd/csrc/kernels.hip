@@ -2505,10 +2505,12 @@ __global__ void k_sino_rows_T(const float* __restrict__ Rc, float* __restrict__ 
     for (int x = threadIdx.x; x < sp.N0; x += blockDim.x) dst[x] = line[x + lb];
 }
 
-// Transpose of k_gather: per tile, the block clears an LDS copy of the source
-// box, adds every point's value times its tap weights into it (LDS atomics),
-// and adds the box into the destination grid (global atomics: neighbouring
-// boxes overlap).  Same tiles, logical block order and clamps as k_gather.
+// Transpose of k_gather for the tiles without a colouring (k_scatter_col has
+// the others): a block per tile group that holds one (g.plain) and slices; it
+// clears an LDS copy of the source box, adds every point's value times its tap
+// weights into it (LDS atomics), and stages the box or adds it into the
+// destination grid (global atomics: neighbouring boxes overlap).  Same tiles
+// and clamps as k_gather.
 template <int KIND>
 __global__ void __launch_bounds__(kGatherThreads) k_scatter(Scatter g, const GTile* __restrict__ tiles) {
     extern __shared__ float box[];
@@ -2516,10 +2518,7 @@ __global__ void __launch_bounds__(kGatherThreads) k_scatter(Scatter g, const GTi
     const int nt = blockDim.x;
     const int nzg = (g.nz + g.zgroup - 1) / g.zgroup;
     const int lbk = xcd_block(blockIdx.x, gridDim.x);
-    const int ng = gridDim.x / nzg;
-    // (with colours: the groups that hold an uncoloured tile; k_scatter_col handles the coloured ones)
-    const int zg = lbk % nzg;
-    const int tile = g.perm ? g.plain[lbk / nzg] : (int)(((long long)(lbk / nzg) * g.tstride) % ng);
+    const int zg = lbk % nzg, tile = g.plain[lbk / nzg];
     const GTile* tb = tiles + (size_t)tile * g.group;
     const GTile t0 = tb[0];
     const int npts = t0.nr * t0.nc;
@@ -2549,7 +2548,7 @@ __global__ void __launch_bounds__(kGatherThreads) k_scatter(Scatter g, const GTi
             if (threadIdx.x + e * nt >= npts) val[e] = 0.f;
         for (int gi = 0; gi < g.group; ++gi) {
             const GTile t = tb[gi];
-            if (t.bw <= 0 || (g.perm && t.cr > 0)) continue;   // uniform over the block
+            if (t.bw <= 0 || t.cr > 0) continue;   // uniform over the block
             const int bs = t.bs;
             const int nbox = bs * t.bh;
             const float2* cbase = g.coord + (size_t)t.span * g.c_span;
@@ -2563,7 +2562,7 @@ __global__ void __launch_bounds__(kGatherThreads) k_scatter(Scatter g, const GTi
             for (int i = threadIdx.x; i < nbox; i += nt) box[i] = 0.f;
             __syncthreads();
             // one point's 16 (4) weighted taps into the box, atomically
-            auto deposit = [&](int e, bool atomic) {
+            auto deposit = [&](int e) {
                 const float2 c = cc[e];
                 float fx = floorf(c.x), fy = floorf(c.y);
                 float ax = c.x - fx, ay = c.y - fy;
@@ -2571,10 +2570,6 @@ __global__ void __launch_bounds__(kGatherThreads) k_scatter(Scatter g, const GTi
                 int ly = min(max((int)fy - 1 - t.y0, 0), t.bh - 4);
                 float* q = box + ly * bs + lx;
                 const float v = val[e];
-                auto add = [&](float* a, float w) {
-                    if (atomic) atomicAdd(a, w);
-                    else *a += w;
-                };
                 if (g.cubic) {
                     float wx[4], wy[4];
                     bspline_w(ax, wx);
@@ -2583,25 +2578,23 @@ __global__ void __launch_bounds__(kGatherThreads) k_scatter(Scatter g, const GTi
                     for (int b = 0; b < 4; ++b) {
                         float vb = wy[b] * v;
 #pragma unroll
-                        for (int a2 = 0; a2 < 4; ++a2) add(q + b * bs + a2, wx[a2] * vb);
+                        for (int a2 = 0; a2 < 4; ++a2) atomicAdd(q + b * bs + a2, wx[a2] * vb);
                     }
                 } else {
                     float* q1 = q + bs + 1;
                     float* q2 = q1 + bs;
-                    add(q1, (1.f - ay) * (1.f - ax) * v);
-                    add(q1 + 1, (1.f - ay) * ax * v);
-                    add(q2, ay * (1.f - ax) * v);
-                    add(q2 + 1, ay * ax * v);
+                    atomicAdd(q1, (1.f - ay) * (1.f - ax) * v);
+                    atomicAdd(q1 + 1, (1.f - ay) * ax * v);
+                    atomicAdd(q2, ay * (1.f - ax) * v);
+                    atomicAdd(q2 + 1, ay * ax * v);
                 }
             };
-            {
 #pragma unroll
-                for (int e = 0; e < PPT; ++e) {
-                    int p = threadIdx.x + e * nt;
-                    if (p < npts && val[e] != 0.f && cc[e].x == cc[e].x) deposit(e, true);
-                }
-                __syncthreads();
+            for (int e = 0; e < PPT; ++e) {
+                int p = threadIdx.x + e * nt;
+                if (p < npts && val[e] != 0.f && cc[e].x == cc[e].x) deposit(e);
             }
+            __syncthreads();
             const float inv = 1.0f / (float)t.bw;
             const int nb = t.bw * t.bh;
             if (g.stage) {
@@ -2801,16 +2794,14 @@ void launch_scatter(const Scatter& g0, const GTile* tiles, int ntiles, int kind,
     g.zgroup = fit_slices(g.zgroup, g.nz, ng, kFitScatter);
     dim3 grid(ng * ((g.nz + g.zgroup - 1) / g.zgroup));
     size_t lds = (size_t)g.box_floats * sizeof(float);
-    if (g.perm) {
-        switch (kind) {
-            case 0: hipLaunchKernelGGL(k_scatter_col<0>, grid, dim3(kScatterThreads), lds, s, g, tiles); break;
-            case 1: hipLaunchKernelGGL(k_scatter_col<1>, grid, dim3(kScatterThreads), lds, s, g, tiles); break;
-            case 2: hipLaunchKernelGGL(k_scatter_col<2>, grid, dim3(kScatterThreads), lds, s, g, tiles); break;
-            default: hipLaunchKernelGGL(k_scatter_col<3>, grid, dim3(kScatterThreads), lds, s, g, tiles); break;
-        }
-        if (g.nplain <= 0) return;
-        grid.x = g.nplain * ((g.nz + g.zgroup - 1) / g.zgroup);
+    switch (kind) {
+        case 0: hipLaunchKernelGGL(k_scatter_col<0>, grid, dim3(kScatterThreads), lds, s, g, tiles); break;
+        case 1: hipLaunchKernelGGL(k_scatter_col<1>, grid, dim3(kScatterThreads), lds, s, g, tiles); break;
+        case 2: hipLaunchKernelGGL(k_scatter_col<2>, grid, dim3(kScatterThreads), lds, s, g, tiles); break;
+        default: hipLaunchKernelGGL(k_scatter_col<3>, grid, dim3(kScatterThreads), lds, s, g, tiles); break;
     }
+    if (g.nplain <= 0) return;
+    grid.x = g.nplain * ((g.nz + g.zgroup - 1) / g.zgroup);
     switch (kind) {
         case 0: hipLaunchKernelGGL(k_scatter<0>, grid, dim3(kGatherThreads), lds, s, g, tiles); break;
         case 1: hipLaunchKernelGGL(k_scatter<1>, grid, dim3(kGatherThreads), lds, s, g, tiles); break;

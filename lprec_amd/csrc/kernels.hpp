@@ -242,7 +242,7 @@ struct Scatter {
     const int* box_off;
     const unsigned short* perm;   // colour-sorted points of the tiles (GTile.pbase)
     const int* cls;               // colour class bounds (GTile.cbase)
-    const int* plain;             // with perm: the nplain tile groups that hold an uncoloured tile
+    const int* plain;             // the nplain tile groups that hold an uncoloured tile
     int nplain;
 };
 // Destination of staged scatter boxes: dst tiles of 32 x 32 points, each the
