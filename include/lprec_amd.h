@@ -187,6 +187,8 @@ int lp_debug_rtc_names(int N, int P0, int Ns, int filter, int cols_threads, int 
 /* Compiles such passes (at most 32, one per line) for gfx950 as a handle does;
  * bit i of *compiled is set when pass i has code.  No device needed. */
 int lp_debug_rtc_compile(const char* names, unsigned* compiled);
+/* The passes compiled so far in this process (each one once). */
+int lp_debug_rtc_passes(void);
 
 #ifdef __cplusplus
 }

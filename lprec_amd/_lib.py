@@ -26,6 +26,7 @@ EXPORTS = (
     "lp_create", "lp_init_fwd", "lp_init_adj", "lp_fwd", "lp_adj", "lp_fwd_T", "lp_adj_T", "lp_destroy",
     "lp_last_error", "lp_mem_info", "lp_info", "lp_set_tuning", "lp_get_tuning",
     "lp_profile", "lp_profile_read", "lp_debug_stop", "lp_debug_copy", "lp_debug_rtc_names", "lp_debug_rtc_compile",
+    "lp_debug_rtc_passes",
     "lp_stream_bench", "lp_fwd_noalloc",
 )
 
@@ -76,6 +77,7 @@ def load():
         "lp_debug_copy": (i32, [vp, i32, vp, ctypes.c_size_t]),
         "lp_debug_rtc_names": (i32, [i32, i32, i32, i32, i32, i32, ctypes.c_char_p, i32]),
         "lp_debug_rtc_compile": (i32, [ctypes.c_char_p, ctypes.POINTER(ctypes.c_uint)]),
+        "lp_debug_rtc_passes": (i32, []),
         "lp_stream_bench": (i32, [i32, vp, vp, ctypes.c_size_t, i32, i32, vp]),
     }
     for name, (res, args) in sig.items():

@@ -809,7 +809,7 @@ int polar_transpose_tables(lp_handle* h, const std::vector<float2>& p2lp, const 
 // N0 = 2048) the generic mixed-radix kernels spend most of their time on run-
 // time index arithmetic.  rtc_build instantiates rtc_kernels.hpp (the same
 // passes with every size a template argument) for this handle's lengths and
-// radix sequences with hipRTC, once per process and set of lengths, and loads
+// radix sequences with hipRTC, once per process and pass, and loads
 // the code object on the handle's device.  Failure is not an error: the
 // generic kernel stays in use for that pass (LPREC_AMD_VERBOSE=1 prints why).
 
@@ -822,26 +822,26 @@ std::string csrc_dir() {
     return (k == std::string::npos ? std::string(".") : p.substr(0, k)) + "/csrc";
 }
 
+// One compiled program, and a pass in it under its mangled name.
 struct RtcCode {
     std::vector<char> code;
-    std::vector<std::string> lowered;
+};
+struct RtcPass {
+    std::shared_ptr<RtcCode> code;
+    std::string lowered;
 };
 std::mutex g_rtc_mu;
-std::map<std::string, std::shared_ptr<RtcCode>> g_rtc_cache;
+std::map<std::string, RtcPass> g_rtc_cache;   // by architecture and instantiation
 
-std::shared_ptr<RtcCode> rtc_compile(const std::string& arch, const std::vector<std::string>& names, std::string& err) {
-    std::string key = arch;
-    for (const auto& n : names) key += ";" + n;
-    std::lock_guard<std::mutex> lock(g_rtc_mu);
-    auto it = g_rtc_cache.find(key);
-    if (it != g_rtc_cache.end()) return it->second;
+// (under g_rtc_mu) compiles the named passes as one program into the cache
+bool rtc_compile(const std::string& arch, const std::vector<std::string>& names, std::string& err) {
     const std::string dir = csrc_dir();
-    if (dir.empty()) { err = "cannot locate the device sources"; return nullptr; }
+    if (dir.empty()) { err = "cannot locate the device sources"; return false; }
     const std::string src = "#include \"rtc_kernels.hpp\"\n";
     hiprtcProgram prog;
     if (hiprtcCreateProgram(&prog, src.c_str(), "lprec_rtc.hip", 0, nullptr, nullptr) != HIPRTC_SUCCESS) {
         err = "hiprtcCreateProgram failed";
-        return nullptr;
+        return false;
     }
     for (const auto& n : names) hiprtcAddNameExpression(prog, n.c_str());
     const std::string a = "--offload-arch=" + arch, inc = "-I" + dir;
@@ -855,47 +855,60 @@ std::shared_ptr<RtcCode> rtc_compile(const std::string& arch, const std::vector<
         if (n) hiprtcGetProgramLog(prog, &log[0]);
         err = "hipRTC compile failed: " + log.substr(0, 2000);
         hiprtcDestroyProgram(&prog);
-        return nullptr;
+        return false;
     }
-    auto out = std::make_shared<RtcCode>();
+    std::vector<std::string> lowered;
     for (const auto& n : names) {
         const char* low = nullptr;
         if (hiprtcGetLoweredName(prog, n.c_str(), &low) != HIPRTC_SUCCESS || !low) {
             err = "no lowered name for " + n;
             hiprtcDestroyProgram(&prog);
-            return nullptr;
+            return false;
         }
-        out->lowered.emplace_back(low);
+        lowered.emplace_back(low);
     }
+    auto out = std::make_shared<RtcCode>();
     size_t cs = 0;
     hiprtcGetCodeSize(prog, &cs);
     out->code.resize(cs);
     if (!cs || hiprtcGetCode(prog, out->code.data()) != HIPRTC_SUCCESS) {
         err = "hiprtcGetCode failed";
         hiprtcDestroyProgram(&prog);
-        return nullptr;
+        return false;
     }
     hiprtcDestroyProgram(&prog);
-    g_rtc_cache[key] = out;
-    return out;
+    for (size_t i = 0; i < names.size(); ++i) g_rtc_cache[arch + ";" + names[i]] = {out, lowered[i]};
+    return true;
 }
 
-// The programs of the named passes: one for all of them (they share the time
-// to read the headers: 1.85 s for the four of N = 2064, 2.25 s one by one), or,
+// The programs that hold the named passes.  A pass is compiled once per
+// process: the plans depend on the batch and the angles, but handles of the
+// same lengths share most passes (as one cache entry per set of passes, a
+// handle of N = 2064 for another batch compiled all four again where one
+// differs).  Those that are missing are one program (they share the time to
+// read the headers: 1.85 s for the four of N = 2064, 2.25 s one by one), or,
 // when that does not compile, one for each pass that does.
 struct RtcProgram {
     std::shared_ptr<RtcCode> code;
-    std::vector<size_t> at;   // the passes in it
+    std::vector<size_t> at;             // the passes in it
+    std::vector<std::string> lowered;   // and their mangled names
 };
 std::vector<RtcProgram> rtc_programs(const std::string& arch, const std::vector<std::string>& names, std::string& err) {
+    std::lock_guard<std::mutex> lock(g_rtc_mu);
+    std::vector<std::string> missing;
+    for (const auto& n : names)
+        if (!g_rtc_cache.count(arch + ";" + n) && std::find(missing.begin(), missing.end(), n) == missing.end()) missing.push_back(n);
+    if (!missing.empty() && !rtc_compile(arch, missing, err))
+        for (size_t i = 0; missing.size() > 1 && i < missing.size(); ++i) rtc_compile(arch, {missing[i]}, err);
     std::vector<RtcProgram> out;
-    if (auto code = rtc_compile(arch, names, err)) {
-        out.push_back({code, {}});
-        for (size_t i = 0; i < names.size(); ++i) out[0].at.push_back(i);
-        return out;
+    for (size_t i = 0; i < names.size(); ++i) {
+        auto it = g_rtc_cache.find(arch + ";" + names[i]);
+        if (it == g_rtc_cache.end()) continue;
+        auto g = std::find_if(out.begin(), out.end(), [&](const RtcProgram& q) { return q.code == it->second.code; });
+        if (g == out.end()) g = out.insert(g, RtcProgram{it->second.code, {}, {}});
+        g->at.push_back(i);
+        g->lowered.push_back(it->second.lowered);
     }
-    for (size_t i = 0; names.size() > 1 && i < names.size(); ++i)
-        if (auto code = rtc_compile(arch, {names[i]}, err)) out.push_back({code, {i}});
     return out;
 }
 
@@ -1215,7 +1228,7 @@ void rtc_build(lp_handle* h) {
         for (size_t i = 0; i < g.at.size(); ++i) {
             const std::string& n = p.names[g.at[i]];
             hipFunction_t f = nullptr;
-            if (hipModuleGetFunction(&f, mod, g.code->lowered[i].c_str()) != hipSuccess) {
+            if (hipModuleGetFunction(&f, mod, g.lowered[i].c_str()) != hipSuccess) {
                 (void)hipGetLastError();
                 p.err = "hipModuleGetFunction failed for " + n;
                 continue;
@@ -2211,6 +2224,11 @@ int lp_debug_rtc_compile(const char* names, unsigned* compiled) {
     for (const RtcProgram& g : rtc_programs("gfx950", list, err))
         for (size_t i : g.at) *compiled |= 1u << i;
     return LP_OK;
+}
+
+int lp_debug_rtc_passes(void) {
+    std::lock_guard<std::mutex> lock(g_rtc_mu);
+    return (int)g_rtc_cache.size();
 }
 
 int lp_get_tuning(const lp_handle* h, int key, int* value) {
