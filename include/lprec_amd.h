@@ -141,7 +141,7 @@ int lp_info(const lp_handle* h, int64_t* info);
  * mask (bit 1: their index arithmetic is redone per slice instead of held in
  * registers, above 256 points; bit 2: registers budgeted for up to 4 waves
  * per SIMD, as many as the blocks' LDS admits, instead of 2; bits 0 and 3
- * have no effect; default 14; recompiles), key 13 = slices per block of
+ * are accepted and have no effect; default 6; recompiles), key 13 = slices per block of
  * lp_fwd's log-polar -> polar gather (>= 1, default 4, halved like key 3; each
  * block reads its tile's coordinates once), key 14 = lp_fwd's image -> log-polar gather
  * reads every tap from global memory, one thread per point (1), instead of

@@ -62,8 +62,8 @@ FftPlan make_plan(int M) {
 
 }  // namespace
 
-// default variant of the compiled passes (lp_handle::rtc_cols_var)
-constexpr int kRtcVar = 14;
+// default variant of the compiled passes (lp_handle::rtc_cols_var): both bits that have an effect
+constexpr int kRtcVar = 6;
 
 struct lp_handle {
     int device = 0;
@@ -91,7 +91,8 @@ struct lp_handle {
     int rtc_mode = 1;
     int rtc_cols_req = 0;   // threads of the compiled column pass (0: automatic)
     // variant of the compiled passes: index arithmetic redone per slice (bit
-    // 1), at least 4 waves per SIMD (bit 2); bits 0 and 3 have no effect
+    // 1), registers for up to 4 waves per SIMD (bit 2); bits 0 and 3 are accepted
+    // and have no effect
     int rtc_cols_var = kRtcVar;
     bool rtc_tried = false;       // with the current settings ...
     bool rtc_pair_tried = false;  // ... and the filtered pair pass
