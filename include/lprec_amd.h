@@ -108,7 +108,10 @@ int lp_stream_bench(int device, float* dst, const float* src, size_t n_floats, i
 int lp_info(const lp_handle* h, int64_t* info);
 /* Kernel schedule knobs: key 0 = log-polar rows per row-FFT block (1..16),
  * key 1 = slices per block in the row/column passes (>=1; halved on launch
- * while a pass would have fewer than 2048 blocks), key 2 = rows per
+ * while a pass would have fewer than 2048 blocks, 768 in the inverse row pass
+ * with 32 elements per lane; the streaming column pass, at Nrho a power of two
+ * from 256 to 8192, takes columns instead, three per slice but at most 6 below
+ * Nrho = 4096, halved below 2048 blocks, 1024 at Nrho = 8192), key 2 = rows per
  * prefilter column chunk (32, 64 or 128), key 3 = slices per block in the
  * tiled gathers and scatters (>=1; halved on launch while there would be too
  * few blocks, each kind by its own count), key 4 = FFT kernel family (1 = radix-16 register

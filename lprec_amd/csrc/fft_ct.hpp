@@ -1,8 +1,8 @@
 // Workgroup FFTs with every size known at compile time, for kernels that the
 // library compiles at run time (hipRTC) for the transform lengths of a handle
-// that the radix-16 register kernels do not cover: lengths with odd factors
-// (2064 = 2^4 3 43 for a centre offset at N0 = 2048), short ones (h < 256) and
-// long ones (rho 8192 at N0 = 4096).
+// that the register kernels do not cover: lengths with odd factors (2064 = 2^4
+// 3 43 for a centre offset at N0 = 2048) and short ones (rows below 256 points,
+// columns below 256).
 //
 // A self-sorting Stockham FFT of NL lines.  Each stage reads its inputs into
 // registers, transforms them, and writes them to the next stage's slots of
@@ -12,10 +12,11 @@
 // one, so loads from HBM, the product with the kernel spectrum and stores to
 // HBM cost no LDS pass of their own.
 //
-// Radices up to 32 run one butterfly per lane in registers (composites as
-// products of small closed forms; 7, 11 and 13 by conjugate pairs); a length
-// costs about the same VALU work per point in each stage whatever its radix,
-// so the host picks few stages of large radix.  A prime factor R >= 17 is a
+// Radices up to 24 without a prime factor above 13 run one butterfly per lane
+// in registers (composites as products of small closed forms; 7, 11 and 13 by
+// conjugate pairs; larger ones would spill); a length costs about the same VALU
+// work per point in each stage whatever its radix, so the host picks few stages
+// of large radix.  A prime factor R >= 17 is a
 // product with the R x R DFT matrix and runs on the matrix cores
 // (mfma_stage): in registers it would cost ~R / 2 fused multiply-adds per
 // point plus as many LDS reads of its weights, which bounded these passes

@@ -939,7 +939,12 @@ double ct_radix_ops(int r) {
 // their radix, so few large ones win, as long as a thread's butterflies of a
 // stage fit in registers -- 24 points -- and the butterflies fill the
 // threads), times the rounds that the waves of all blocks take over the
-// chip.  Prime factors >= 17 are matrix-core stages and come first (no
+// chip.  (Some column plans still spill 20 - 24 of the 128 registers that four
+// waves per SIMD leave: 18 8 8 at N = 576, 16 14 12 at 1344, 22 18 8 at 1584, 20
+// 20 8 at 1600, 22 20 20 at 4400; the estimate does not see it.  fwd at these
+// lengths, 8 slices, with the earlier compiled passes (radices up to 8 and odd
+// ones with their weights in LDS) and with these: 232 / 164, 1492 / 801, 2736 /
+// 1164, 1906 / 1166 us; 4400, 1 slice 2451 / 1334.)  Prime factors >= 17 are matrix-core stages and come first (no
 // twiddles), then the odd radices (their strided LDS writes spread over the
 // banks).  Waves that share a CU hide each other's latency, up to 16 (128
 // registers).  Measured against the neighbours of its choices (32 slices):
