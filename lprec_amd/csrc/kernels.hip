@@ -2005,31 +2005,34 @@ size_t rows_lds_bytes(int ldm, int R) { return (size_t)lds_slots(R * ldm) * size
 size_t cols_lds_bytes(int M) { return (size_t)lds_slots(M) * sizeof(float2); }
 size_t sino_lds_bytes(int Lh, int N) { return (size_t)lds_slots(Lh) * sizeof(float2) + (size_t)(2 * N) * sizeof(float); }
 
-// dynamic LDS above 64 KiB (gfx950 has 160 KiB per workgroup) is opted into
-// per kernel; a refusal surfaces as a launch error in check_launch
+// Dynamic LDS above 64 KiB (gfx950 has 160 KiB per workgroup) is opted into
+// per kernel.  False when it and the kernel's static LDS exceed the limit: the
+// kernel is then not launched (its dispatch would abort the process), and the
+// error reaches the caller through check_launch.
 template <class K>
-static void allow_lds(K k, size_t bytes) {
-    if (bytes > 65536) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+static bool allow_lds(K k, size_t bytes) {
+    return bytes <= 65536 || hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes) == hipSuccess;
 }
+constexpr size_t kLdsLimit = 160 * 1024;
 
 #define LP_DISPATCH_EPT(ept, KER, grid, block, lds, stream, ...)                                   \
     do {                                                                                          \
         switch (ept) {                                                                            \
-            case 4: allow_lds(KER<4>, lds); hipLaunchKernelGGL(KER<4>, grid, block, lds, stream, __VA_ARGS__); break;   \
-            case 8: allow_lds(KER<8>, lds); hipLaunchKernelGGL(KER<8>, grid, block, lds, stream, __VA_ARGS__); break;   \
-            case 16: allow_lds(KER<16>, lds); hipLaunchKernelGGL(KER<16>, grid, block, lds, stream, __VA_ARGS__); break; \
-            default: allow_lds(KER<32>, lds); hipLaunchKernelGGL(KER<32>, grid, block, lds, stream, __VA_ARGS__); break; \
+            case 4: if (allow_lds(KER<4>, lds)) hipLaunchKernelGGL(KER<4>, grid, block, lds, stream, __VA_ARGS__); break;   \
+            case 8: if (allow_lds(KER<8>, lds)) hipLaunchKernelGGL(KER<8>, grid, block, lds, stream, __VA_ARGS__); break;   \
+            case 16: if (allow_lds(KER<16>, lds)) hipLaunchKernelGGL(KER<16>, grid, block, lds, stream, __VA_ARGS__); break; \
+            default: if (allow_lds(KER<32>, lds)) hipLaunchKernelGGL(KER<32>, grid, block, lds, stream, __VA_ARGS__); break; \
         }                                                                                         \
     } while (0)
 
 #define LP_DISPATCH_EPT2(ept, KER, B, grid, block, lds, stream, ...)                                                    \
     do {                                                                                                             \
         switch (ept) {                                                                                               \
-            case 4: allow_lds(KER<4, B>, lds); hipLaunchKernelGGL((KER<4, B>), grid, block, lds, stream, __VA_ARGS__); break;   \
-            case 8: allow_lds(KER<8, B>, lds); hipLaunchKernelGGL((KER<8, B>), grid, block, lds, stream, __VA_ARGS__); break;   \
-            case 16: allow_lds(KER<16, B>, lds); hipLaunchKernelGGL((KER<16, B>), grid, block, lds, stream, __VA_ARGS__); break; \
-            default: allow_lds(KER<32, B>, lds); hipLaunchKernelGGL((KER<32, B>), grid, block, lds, stream, __VA_ARGS__); break; \
+            case 4: if (allow_lds(KER<4, B>, lds)) hipLaunchKernelGGL((KER<4, B>), grid, block, lds, stream, __VA_ARGS__); break;   \
+            case 8: if (allow_lds(KER<8, B>, lds)) hipLaunchKernelGGL((KER<8, B>), grid, block, lds, stream, __VA_ARGS__); break;   \
+            case 16: if (allow_lds(KER<16, B>, lds)) hipLaunchKernelGGL((KER<16, B>), grid, block, lds, stream, __VA_ARGS__); break; \
+            default: if (allow_lds(KER<32, B>, lds)) hipLaunchKernelGGL((KER<32, B>), grid, block, lds, stream, __VA_ARGS__); break; \
         }                                                                                                            \
     } while (0)
 
@@ -2139,14 +2142,24 @@ static size_t rows16_lds(const RowPass& rp) {
 #define LP_DISPATCH_MID(mid, KER, grid, block, lds, stream, ...)                                                  \
     do {                                                                                                         \
         switch (mid) {                                                                                           \
-            case 1: allow_lds(KER<1>, lds); hipLaunchKernelGGL(KER<1>, grid, block, lds, stream, __VA_ARGS__); break;   \
-            case 2: allow_lds(KER<2>, lds); hipLaunchKernelGGL(KER<2>, grid, block, lds, stream, __VA_ARGS__); break;   \
-            case 4: allow_lds(KER<4>, lds); hipLaunchKernelGGL(KER<4>, grid, block, lds, stream, __VA_ARGS__); break;   \
-            case 8: allow_lds(KER<8>, lds); hipLaunchKernelGGL(KER<8>, grid, block, lds, stream, __VA_ARGS__); break;   \
-            default: allow_lds(KER<16>, lds); hipLaunchKernelGGL(KER<16>, grid, block, lds, stream, __VA_ARGS__); break; \
+            case 1: if (allow_lds(KER<1>, lds)) hipLaunchKernelGGL(KER<1>, grid, block, lds, stream, __VA_ARGS__); break;   \
+            case 2: if (allow_lds(KER<2>, lds)) hipLaunchKernelGGL(KER<2>, grid, block, lds, stream, __VA_ARGS__); break;   \
+            case 4: if (allow_lds(KER<4>, lds)) hipLaunchKernelGGL(KER<4>, grid, block, lds, stream, __VA_ARGS__); break;   \
+            case 8: if (allow_lds(KER<8>, lds)) hipLaunchKernelGGL(KER<8>, grid, block, lds, stream, __VA_ARGS__); break;   \
+            default: if (allow_lds(KER<16>, lds)) hipLaunchKernelGGL(KER<16>, grid, block, lds, stream, __VA_ARGS__); break; \
         }                                                                                                        \
     } while (0)
 
+
+// Rows per block of the mixed-radix row kernels: at most 8 (their register
+// budget), fewer where the rows and the kernels' static LDS (weights of odd
+// radices and row ranges: 5504 bytes) would pass the limit (8 rows of h = 2400
+// are 163208 bytes).  Nrho stays divisible since R is a power of two.
+static int generic_rows(const RowPass& rp) {
+    int R = std::min(rp.R, 8);
+    while (R > 1 && rows_lds_bytes(rp.ldm, R) + 5504 > kLdsLimit) R /= 2;
+    return R;
+}
 
 // Slices per block, reduced for small batches so that a launch still has
 // enough blocks to fill the chip several times over.
@@ -2164,11 +2177,9 @@ void launch_rows_fwd(const RowPass& rp0, const float* F, const int2* range, hipS
         LP_DISPATCH_MID(mid, k_rows16_fwd, grid, block, rows16_lds(rp), s, rp, F, range);
         return;
     }
-    // the mixed-radix kernels keep at most 8 rows per block (their register
-    // budget); Nrho stays divisible since R is a power of two
     RowPass rg = rp;
     // the compiled pass has its rows per block built in
-    rg.R = rg.rtc_rows_fwd ? rg.rtc_R : std::min(rg.R, 8);
+    rg.R = rg.rtc_rows_fwd ? rg.rtc_R : generic_rows(rg);
     rg = fit_zgroup(rg, 3LL * (rg.Nrho / rg.R));
     dim3 grid(rg.Nrho / rg.R, 3, (rg.nz + rg.zgroup - 1) / rg.zgroup);
     if (rg.rtc_rows_fwd) {
@@ -2215,11 +2226,11 @@ void launch_rows_inv(const RowPass& rp0, float* G, const int2* wrange, hipStream
             const RowPass rq = fit_zgroup(rp0, 3LL * (rp0.Nrho / rp0.R), 768);
             const dim3 g((rq.Nrho / rq.R) * 3 * ((rq.nz + rq.zgroup - 1) / rq.zgroup));
             if (rq.h == 1024) {
-                allow_lds(k_rows32_inv<1024>, RowsWave<1024>::lds);
-                hipLaunchKernelGGL(k_rows32_inv<1024>, g, dim3(512), RowsWave<1024>::lds, s, rq, G, wrange);
+                if (allow_lds(k_rows32_inv<1024>, RowsWave<1024>::lds))
+                    hipLaunchKernelGGL(k_rows32_inv<1024>, g, dim3(512), RowsWave<1024>::lds, s, rq, G, wrange);
             } else {
-                allow_lds(k_rows32_inv<2048>, RowsWave<2048>::lds);
-                hipLaunchKernelGGL(k_rows32_inv<2048>, g, dim3(512), RowsWave<2048>::lds, s, rq, G, wrange);
+                if (allow_lds(k_rows32_inv<2048>, RowsWave<2048>::lds))
+                    hipLaunchKernelGGL(k_rows32_inv<2048>, g, dim3(512), RowsWave<2048>::lds, s, rq, G, wrange);
             }
             return;
         }
@@ -2228,7 +2239,7 @@ void launch_rows_inv(const RowPass& rp0, float* G, const int2* wrange, hipStream
         return;
     }
     RowPass rg = rp;
-    rg.R = rg.rtc_rows_inv ? rg.rtc_R : std::min(rg.R, 8);
+    rg.R = rg.rtc_rows_inv ? rg.rtc_R : generic_rows(rg);
     rg = fit_zgroup(rg, 3LL * (rg.Nrho / rg.R));
     dim3 grid(rg.Nrho / rg.R, 3, (rg.nz + rg.zgroup - 1) / rg.zgroup);
     if (rg.rtc_rows_inv) {
