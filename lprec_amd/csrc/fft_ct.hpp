@@ -13,10 +13,10 @@
 // HBM cost no LDS pass of their own.
 //
 // Radices up to 24 without a prime factor above 13 run one butterfly per lane
-// in registers (composites as products of small closed forms; 7, 11 and 13 by
-// conjugate pairs; larger ones would spill); a length costs about the same VALU
-// work per point in each stage whatever its radix, so the host picks few stages
-// of large radix.  A prime factor R >= 17 is a
+// in registers (composites as coprime products of small closed forms, without
+// twiddles; 7, 11 and 13 by conjugate pairs; larger ones would spill); a length
+// costs about the same VALU work per point in each stage whatever its radix, so
+// the host picks few stages of large radix.  A prime factor R >= 17 is a
 // product with the R x R DFT matrix and runs on the matrix cores
 // (mfma_stage): in registers it would cost ~R / 2 fused multiply-adds per
 // point plus as many LDS reads of its weights, which bounded these passes
@@ -75,10 +75,17 @@ constexpr int largest_prime(int n) {
         while (n % q == 0) { p = q; n /= q; }
     return p;
 }
-// the first factor of a composite register radix
+// the first factor of a composite register radix: coprime to the other one
+// unless the radix is a prime power
 constexpr int split_of(int R) {
-    return R % 13 == 0 ? 13 : R % 11 == 0 ? 11 : R % 7 == 0 ? 7 : R % 5 == 0 ? 5 : R % 9 == 0 ? 3
+    return R == 9 ? 3 : R % 13 == 0 ? 13 : R % 11 == 0 ? 11 : R % 7 == 0 ? 7 : R % 5 == 0 ? 5 : R % 9 == 0 ? 9
            : R % 8 == 0 ? 8 : R % 4 == 0 ? 4 : R % 3 == 0 ? 3 : 2;
+}
+// the multiple of B below A B that is 1 mod A (A, B coprime)
+constexpr int idempotent(int A, int B) {
+    int e = B;
+    while (e % A != 1) e += B;
+    return e;
 }
 // a stage on the matrix cores
 constexpr bool on_mfma(int R) { return R >= 17 && largest_prime(R) == R; }
@@ -125,30 +132,53 @@ __device__ __forceinline__ void dft(float2* v, int dir) {
     } else if constexpr (largest_prime(R) == R) {
         dft_odd<R>(v, dir);
     } else {
-        // R = A B: A-point DFTs over elements B apart, twiddles, B-point DFTs
         constexpr int A = split_of(R), B = R / A;
-        constexpr Turn<R> w{};
         float2 a[B][A];
+        if constexpr (A % B != 0) {
+            // R = A B, coprime: with input B n1 + A n2 and output k1 mod A, k2 mod
+            // B it is A-point DFTs over n1 and B-point DFTs over n2, without
+            // twiddles (those of 10 and 20, rounded, have mean gains of 5e-9 and
+            // 8e-9, which add up over the passes)
+            constexpr int eA = idempotent(A, B), eB = idempotent(B, A);
 #pragma unroll
-        for (int n2 = 0; n2 < B; ++n2) {
+            for (int n2 = 0; n2 < B; ++n2) {
 #pragma unroll
-            for (int n1 = 0; n1 < A; ++n1) a[n2][n1] = v[n1 * B + n2];
-            dft<A>(a[n2], dir);
+                for (int n1 = 0; n1 < A; ++n1) a[n2][n1] = v[(B * n1 + A * n2) % R];
+                dft<A>(a[n2], dir);
+            }
 #pragma unroll
-            for (int k1 = 1; k1 < A; ++k1)
-                if (n2 > 0) {
-                    const float c = w.c[n2 * k1], s = w.s[n2 * k1];
-                    a[n2][k1] = cmul(a[n2][k1], make_float2(c, dir < 0 ? -s : s));
-                }
-        }
+            for (int k1 = 0; k1 < A; ++k1) {
+                float2 t[B];
 #pragma unroll
-        for (int k1 = 0; k1 < A; ++k1) {
-            float2 t[B];
+                for (int n2 = 0; n2 < B; ++n2) t[n2] = a[n2][k1];
+                dft<B>(t, dir);
 #pragma unroll
-            for (int n2 = 0; n2 < B; ++n2) t[n2] = a[n2][k1];
-            dft<B>(t, dir);
+                for (int k2 = 0; k2 < B; ++k2) v[(eA * k1 + eB * k2) % R] = t[k2];
+            }
+        } else {
+            // 9 = 3 3: DFTs over elements 3 apart, twiddles, DFTs
+            constexpr Turn<R> w{};
 #pragma unroll
-            for (int k2 = 0; k2 < B; ++k2) v[k1 + A * k2] = t[k2];
+            for (int n2 = 0; n2 < B; ++n2) {
+#pragma unroll
+                for (int n1 = 0; n1 < A; ++n1) a[n2][n1] = v[n1 * B + n2];
+                dft<A>(a[n2], dir);
+#pragma unroll
+                for (int k1 = 1; k1 < A; ++k1)
+                    if (n2 > 0) {
+                        const float c = w.c[n2 * k1], s = w.s[n2 * k1];
+                        a[n2][k1] = cmul(a[n2][k1], make_float2(c, dir < 0 ? -s : s));
+                    }
+            }
+#pragma unroll
+            for (int k1 = 0; k1 < A; ++k1) {
+                float2 t[B];
+#pragma unroll
+                for (int n2 = 0; n2 < B; ++n2) t[n2] = a[n2][k1];
+                dft<B>(t, dir);
+#pragma unroll
+                for (int k2 = 0; k2 < B; ++k2) v[k1 + A * k2] = t[k2];
+            }
         }
     }
 }
@@ -207,11 +237,26 @@ __device__ __forceinline__ Source<Get, Fix> make_source(Get g, Fix f) {
 // (first version of these stages: 70 % of the wave cycles waiting).
 __device__ __forceinline__ void issue_loads() { __builtin_amdgcn_sched_barrier(0); }
 
-constexpr int log2_ceil(int r) {
-    int n = 0;
-    while ((1 << n) < r) ++n;
-    return n;
-}
+// The powers w^q, q < R, of a butterfly's twiddle from few table reads: w .. w^m
+// and w^b at steps of 2 m + 1 (the last one at R - 1), every other one the product
+// of a w^b with w^d or its conjugate, d <= m.  As many reads as for w, w^2, w^4, ..
+// up to radix 13 (one more above), whose products of up to four factors round
+// worse: with these powers and the twiddle-free radices above, fwd and adj at 38
+// lengths from 96 to 2000 are on average 0.94 as far from float64, in the same time.
+template <int R>
+struct Powers {
+    static constexpr int steps(int m) { return R - 1 > m ? (R - 1 - m + 2 * m) / (2 * m + 1) : 0; }
+    static constexpr int pick() {
+        int m = 1;
+        for (int k = 2; k < 4; ++k)
+            if (k + steps(k) < m + steps(m)) m = k;
+        return m;
+    }
+    static constexpr int m = pick(), count = R > 1 ? m + steps(m) : 1;
+    // nearest power that is read, and the slot of a power that is
+    static constexpr int base(int q) { return q <= m ? q : (q + m) / (2 * m + 1) * (2 * m + 1) < R ? (q + m) / (2 * m + 1) * (2 * m + 1) : R - 1; }
+    static constexpr int slot(int q) { return q <= m ? q - 1 : m + (q + m) / (2 * m + 1) - 1; }
+};
 
 // One register stage of radix R (Ns = product of the radices before it) over
 // NL lines of M points: in (a Source) gives the inputs, the post operation on the
@@ -222,16 +267,17 @@ constexpr int log2_ceil(int r) {
 template <int M, int NL, int NT, int Ns, int R, bool MID, class In, class P, class Out>
 __device__ __forceinline__ void reg_stage(In in, P post, Out out, const float2* __restrict__ tw, int dir, int tid) {
     constexpr int nbf = M / R, total = NL * nbf, NI = (total + NT - 1) / NT;
-    constexpr int tstep = M / (Ns * R), LW = log2_ceil(R);
-    float2 v[NI][R], wl[NI][LW > 0 ? LW : 1];
+    constexpr int tstep = M / (Ns * R);
+    using W = Powers<R>;
+    float2 v[NI][R], wl[NI][W::count];
     auto item = [&](int c) { return (c + 1) * NT <= total ? tid + c * NT : min(tid + c * NT, total - 1); };
 #pragma unroll
     for (int c = 0; c < NI; ++c) {
         const int t = item(c), b = NL == 1 ? 0 : t / nbf, i = t - b * nbf;
         if (Ns > 1) {
-            // w, w^2, w^4, ... of the butterfly; the other powers are products
 #pragma unroll
-            for (int l = 0; l < LW; ++l) wl[c][l] = tw[((i % Ns) * tstep) << l];
+            for (int q = 1; q < R; ++q)
+                if (W::base(q) == q) wl[c][W::slot(q)] = tw[(i % Ns) * tstep * q];
         }
 #pragma unroll
         for (int q = 0; q < R; ++q) v[c][q] = in.get(b, i + q * nbf);
@@ -249,11 +295,12 @@ __device__ __forceinline__ void reg_stage(In in, P post, Out out, const float2* 
 #pragma unroll
         for (int q = 0; q < R; ++q) v[c][q] = in.fix(b, i + q * nbf, v[c][q]);
         if (Ns > 1) {
-            float2 w[R > 1 ? R : 2];
 #pragma unroll
             for (int q = 1; q < R; ++q) {
-                w[q] = (q & (q - 1)) == 0 ? (dir < 0 ? wl[c][log2_ceil(q)] : cconj(wl[c][log2_ceil(q)])) : cmul(w[q & (q - 1)], w[q & -q]);
-                v[c][q] = cmul(v[c][q], w[q]);
+                float2 w = wl[c][W::slot(q)];
+                const int d = q - W::base(q);
+                if (d != 0) w = d > 0 ? cmul(w, wl[c][d - 1]) : cmul(w, cconj(wl[c][-d - 1]));
+                v[c][q] = cmul(v[c][q], dir < 0 ? w : cconj(w));
             }
         }
         dft<R>(v[c], dir);
